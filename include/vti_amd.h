@@ -310,7 +310,9 @@ int vti2d_gn_hessian_vepsdel(vti_ctx *ctx, float *gv, float *geps, float *gdel, 
  * vti2d_objfunc_gradient (rate/dt >= 2, (nt-1) % (rate/dt) == 0, ot = 0).
  * levels: time levels advanced per launch, 1 or 2 (0: 2); tile_rows: rows
  * of a two-level workgroup tile, 4, 8 or 16 (0: 16).  Neither changes a bit of
- * the result.  snap_fmt: 0 keeps the imaging snapshots in FP32 (the result
+ * the result.  The default shape (two levels, 16 rows) leaves the choice to the
+ * library: with FP32 or S16 snapshots, shots that fit the chip (up to about
+ * 0.78 M points at once) run resident, all levels of a pass in one launch.  snap_fmt: 0 keeps the imaging snapshots in FP32 (the result
  * then equals the one-shot driver's bit for bit); 1 (FP16) and 2 (BF16)
  * store each snapshot slice scaled by a power of two, 3 (S16) 16-bit
  * integers with a power-of-two scale per 64-point row piece, halving their memory;
@@ -334,7 +336,8 @@ int vti2d_objfunc_gradient_batch(vti_ctx *ctx, double *objfunc, double *gc11, do
  * (an error when the whole does not fit the free device memory), and
  * records each wave's launch sequence -- forward pass and residual, then
  * adjoint pass and FP64 accumulation, every buffer clearing done by a
- * kernel -- into two hipGraphs on the context's stream.
+ * kernel -- into two hipGraphs on the context's stream (waves that run
+ * resident, a few launches each, are enqueued anew by every run instead).
  * vti2d_batch_plan_run uploads c11/c13/c33 and replays the graphs, wave k
  * on the context's stream or (odd k) a second stream the plan holds, each
  * forward pass beside the previous wave's adjoint, and returns what

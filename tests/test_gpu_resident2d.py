@@ -1,0 +1,60 @@
+"""The resident 2D kernels (one launch per pass, every shot's state on the
+chip) against the per-level kernels, which `levels=1` asks for: the same bits
+at the edges of their tiles (64 columns, 4 rows to a wavefront's 6), for ragged
+last tiles, with several receivers in one column, in waves of several shots,
+and through the fallback for a grid that does not fit the chip."""
+import numpy as np
+import pytest
+
+from common2d import layered2d
+from common3d import cij_from, ricker
+
+pytestmark = pytest.mark.gpu
+
+
+def _shots(widths, nz, npad, nt, vertical=False, seed=1):
+    rng = np.random.default_rng(seed)
+    NX = max(widths) + 7
+    nnz = nz + 2 * npad
+    c = cij_from(*layered2d(nnz, NX + 2 * npad, seed))
+    shots, rloc = [], []
+    for w in widths:
+        w2 = w + 2 * npad
+        if vertical:  # a receiver in every interior row of two columns
+            cols = sorted({4, w2 - 5})
+            r = [(x, z) for x in cols for z in range(4, nnz - 4)]
+        else:
+            r = [(x, 4 + (nnz - 8) // 2) for x in range(4, w2 - 4)]
+        shots.append((int(rng.integers(0, NX - w + 1)), w, 4 + (w2 - 8) // 2, 4, len(r), len(rloc)))
+        rloc += r
+    nnt = (nt - 1) // 4 + 1
+    data = (1e-7 * rng.standard_normal(nnt * len(rloc))).astype(np.float32)
+    return data, c, ricker(nt, 1e-3, 25.0, 0.02), np.array(shots, np.int32), np.array(rloc, np.int32), \
+        (NX, nz, nt, npad, 10.0, 10.0, 1e-3, 4e-3)
+
+
+@pytest.mark.parametrize("snap", ["fp32", "s16"])
+@pytest.mark.parametrize("widths,nz,npad,nt,vertical", [
+    ((1,), 1, 4, 9, False),                    # a single interior point
+    ((64,), 4, 4, 21, False),                  # one tile exactly
+    ((65, 67, 128), 5, 4, 29, False),          # last tiles of 1, 3 and 64 columns, 5 rows
+    ((70, 61), 93, 5, 61, True),               # 97 rows: ragged for every row count; receivers down two columns
+    ((200, 90, 131, 64, 177), 60, 12, 81, False),
+    ((500,), 300, 20, 61, False),              # several hundred tiles, the waves still apart (a zero gradient)
+])
+def test_resident_equals_per_level(vti, ctx, widths, nz, npad, nt, vertical, snap):
+    data, c, w, shots, rloc, rest = _shots(widths, nz, npad, nt, vertical)
+    print("resident", widths, nz, npad, nt, snap, flush=True)
+    f0, g0 = vti.objfunc_gradient2d_batch(ctx, data, *c, w, shots, rloc, *rest, levels=1, snap=snap)
+    f1, g1 = vti.objfunc_gradient2d_batch(ctx, data, *c, w, shots, rloc, *rest, snap=snap)
+    assert np.isfinite(g0).all() and f0 > 0 and (nt == 61 or g0.any())
+    assert f0 == f1 and np.array_equal(g0, g1)
+
+
+def test_grid_beyond_the_chip(vti, ctx):
+    """1.2 M points do not fit: the default call then runs the two-level kernels."""
+    data, c, w, shots, rloc, rest = _shots((1500,), 700, 20, 9)
+    print("resident fallback by size", flush=True)
+    f0, g0 = vti.objfunc_gradient2d_batch(ctx, data, *c, w, shots, rloc, *rest, levels=1)
+    f1, g1 = vti.objfunc_gradient2d_batch(ctx, data, *c, w, shots, rloc, *rest)
+    assert f0 == f1 and np.array_equal(g0, g1)

@@ -22,6 +22,7 @@
 #include <vector>
 
 #include "vti2d_batch_kernels.h"
+#include "vti2d_res.h"
 #include "vti_amd.h"
 #include "vti_ctx.h"
 #include "vti_dbuf.h"
@@ -164,6 +165,9 @@ struct ShotIn {
 struct BatchArgs {
     int ns, nr, NX, nz, nt, npad, NNX, nnz, ratio, nnt, nnt_data, levels, BYT, snap_fmt;
     bool half;
+    bool res = false;  // the waves run resident (vti2d_res.h)
+    bool grad = true;  // objective and gradient (false: traces only)
+    const float *wavelet = nullptr;
     float dx2, dz2, dt2;
     std::vector<ShotIn> in;
     std::vector<long long> data_off;
@@ -298,6 +302,8 @@ struct BatchWave {
     DBuf<unsigned short> snaph;
     DBuf<unsigned> amax;
     DBuf<double> part;
+    vti::ResRun res;     // active when the wave runs resident
+    bool level = false;  // a resident wave to be run on the per-level kernels
     // residual partial sums per shot (merged requests): the one-shot
     // driver's block count for each shot's traces, and their offsets in part
     std::vector<int> pblk, poff;
@@ -412,6 +418,45 @@ int pool_alloc(WavePool &pool, const BatchArgs &a, hipStream_t st)
     return rc;
 }
 
+// trace rows and snapshot slots bracketing adjoint level it
+vti::LevelB adjoint_level(const BatchArgs &a, int it)
+{
+    vti::LevelB l;
+    float fr = (float)((it + 1.) / a.ratio);
+    l.row = (int)fr;
+    l.fr = fr - l.row;
+    float f = (float)it / a.ratio;
+    l.slot = (int)f;
+    l.f = f - l.slot;
+    return l;
+}
+
+// What each level of a resident wave does, from the wavelet (snap: with the
+// D snapshots), and the adjoint's levels.
+void res_levels(vti::ResRun &r, const BatchArgs &a, const float *wavelet, bool snap)
+{
+    r.lf.assign(a.nt, vti::LevF{0.f, -1, -1, 0});
+    for (int it = 1; it < a.nt; ++it)
+        r.lf[it] = vti::LevF{a.dt2 * wavelet[it - 1], snap && it > 1 && (it - 1) % a.ratio == 0 ? (it - 1) / a.ratio : -1,
+                             it > 1 && it % a.ratio == 0 ? it / a.ratio : -1, 0};
+    r.lb.clear();
+    if (!snap) return;
+    vti::LevelB first{a.nnt_data - 1, 0.f, 0, (float)((a.nt - 2.) / a.ratio)};  // the first image's slots
+    first.slot = (int)first.f;
+    first.f -= first.slot;
+    r.lb.push_back(first);
+    for (int it = a.nt - 3; it >= 0; --it) r.lb.push_back(adjoint_level(a, it));
+}
+
+// The resident form of a wave (sized): its shape and tables.
+int setup_res(BatchWave &W, const BatchArgs &a, const int *rloc, hipStream_t st)
+{
+    std::vector<int> r0;
+    for (int j = 0; j < W.nw; ++j) r0.push_back(a.in[W.s0 + j].r0);
+    res_levels(W.res, a, a.wavelet, a.grad);
+    return W.res.setup(W.sb, a.nnz, a.snap_fmt, rloc, r0.data(), st);
+}
+
 // Allocate (or, with a pool, view) the wave's device buffers and upload its
 // tables, receiver map and observed data.
 int fill_wave(BatchWave &W, const BatchArgs &a, const float *data, const int *rloc, hipStream_t st,
@@ -419,10 +464,18 @@ int fill_wave(BatchWave &W, const BatchArgs &a, const float *data, const int *rl
 {
     const int s0 = W.s0, nw = W.nw, nnt = a.nnt;
     const int nrec = W.nrec;
+    if (a.res) {
+        const int rc = setup_res(W, a, rloc, st);
+        if (rc) return rc;
+    }
+    // a resident wave needs neither the wavefields nor the receiver map in
+    // memory; one on shared buffers (a plan) has them for the per-level kernels,
+    // should a resident run give up
+    const bool level = !a.res || pool;
     std::vector<long long> fidx(nrec), tb(nrec);
     std::vector<int> tsd(nrec);
-    std::vector<int> hmap((size_t)W.f_total, -1);
-    for (int j = 0, k = 0; j < nw; ++j) {
+    std::vector<int> hmap(level ? (size_t)W.f_total : 0, -1);
+    for (int j = 0, k = 0; level && j < nw; ++j) {
         const ShotIn &q = a.in[s0 + j];
         for (int r = 0; r < q.nr; ++r, ++k) {
             const int x = rloc[2 * (q.r0 + r)], z = rloc[2 * (q.r0 + r) + 1];
@@ -432,20 +485,22 @@ int fill_wave(BatchWave &W, const BatchArgs &a, const float *data, const int *rl
             hmap[(size_t)fidx[k]] = r;
         }
     }
-    std::vector<float> obs_h((size_t)std::max<long long>(W.tr_total, 1));
+    std::vector<float> obs_h((size_t)(a.grad ? std::max<long long>(W.tr_total, 1) : 1));
     for (int j = 0; j < nw; ++j)
-        if (a.in[s0 + j].nr)
+        if (a.grad && a.in[s0 + j].nr)
             std::memcpy(obs_h.data() + W.sb[j].r_off, data + a.data_off[s0 + j],
                         sizeof(float) * (size_t)a.nnt_data * a.in[s0 + j].nr);
     const long long f_total = W.f_total, tr_total = W.tr_total;
     int rc = W.sbd.alloc(nw, st);
-    if (!rc) rc = W.sbtd.alloc(nw, st);
-    if (!rc) rc = W.tsh.alloc(W.tile_shot.size(), st);
-    if (!rc) rc = W.tsht.alloc(W.tile_shot_t.size(), st);
-    if (!rc) rc = W.recmap.alloc((size_t)f_total, st);
-    if (!rc) rc = W.tsdd.alloc(nrec, st);
-    if (!rc) rc = W.fidxd.alloc(nrec, st);
-    if (!rc) rc = W.tbd.alloc(nrec, st);
+    if (level) {
+        if (!rc) rc = W.sbtd.alloc(nw, st);
+        if (!rc) rc = W.tsh.alloc(W.tile_shot.size(), st);
+        if (!rc) rc = W.tsht.alloc(W.tile_shot_t.size(), st);
+        if (!rc) rc = W.recmap.alloc((size_t)f_total, st);
+        if (!rc) rc = W.tsdd.alloc(nrec, st);
+        if (!rc) rc = W.fidxd.alloc(nrec, st);
+        if (!rc) rc = W.tbd.alloc(nrec, st);
+    }
     // snapshot slots 1.. are written by the forward pass before the adjoint
     // reads them; slot 0 (D of the zero level 0) is never written and is
     // cleared by enqueue_wave, so the slots themselves need no clearing
@@ -468,22 +523,22 @@ int fill_wave(BatchWave &W, const BatchArgs &a, const float *data, const int *rl
         }
         W.tr.borrow(pool->tr_b, (size_t)std::max<long long>(tr_total, 1));
     } else {
-        for (int k = 0; k < 4 && !rc; ++k) {
+        for (int k = 0; k < 4 && level && !rc; ++k) {
             rc = W.P[k].alloc((size_t)f_total, st);
             if (!rc) rc = W.Q[k].alloc((size_t)f_total, st);
         }
-        for (int k = 0; k < 3 && !rc; ++k) rc = W.G[k].alloc((size_t)f_total, st);
+        for (int k = 0; k < 3 && a.grad && !rc; ++k) rc = W.G[k].alloc((size_t)f_total, st, false);
         if (a.half) {
             if (!rc) rc = W.snaph.alloc((size_t)W.snap_total, st, false);
             if (!rc && a.snap_fmt != 3) rc = W.stage.alloc((size_t)(2 * f_total), st);
             if (!rc) rc = W.scale.alloc((size_t)wave_scale_count(W, a), st);
             if (!rc) rc = W.amax.alloc((size_t)(2 * nnt * nw), st);
-        } else {
+        } else if (a.grad) {
             if (!rc) rc = W.snapf.alloc((size_t)W.snap_total, st, false);
         }
         if (!rc) rc = W.tr.alloc((size_t)std::max<long long>(tr_total, 1), st);
     }
-    if (!rc) rc = W.obs.alloc((size_t)std::max<long long>(tr_total, 1), st);
+    if (!rc) rc = W.obs.alloc(obs_h.size(), st);
     W.pblk.assign(nw, 0);
     W.poff.assign(nw, 0);
     int ptot = 0;
@@ -495,17 +550,20 @@ int fill_wave(BatchWave &W, const BatchArgs &a, const float *data, const int *rl
     if (!rc) rc = W.part.alloc(std::max(kNblkR, ptot), st);
     if (rc) return rc;
     VTI_HIP(hipMemcpyAsync(W.sbd.p, W.sb.data(), sizeof(ShotB) * nw, hipMemcpyHostToDevice, st));
-    VTI_HIP(hipMemcpyAsync(W.sbtd.p, W.sbt.data(), sizeof(ShotB) * nw, hipMemcpyHostToDevice, st));
-    VTI_HIP(hipMemcpyAsync(W.tsh.p, W.tile_shot.data(), sizeof(int) * W.tile_shot.size(), hipMemcpyHostToDevice, st));
-    VTI_HIP(hipMemcpyAsync(W.tsht.p, W.tile_shot_t.data(), sizeof(int) * W.tile_shot_t.size(),
-                           hipMemcpyHostToDevice, st));
-    VTI_HIP(hipMemcpyAsync(W.recmap.p, hmap.data(), sizeof(int) * hmap.size(), hipMemcpyHostToDevice, st));
-    if (nrec) {
+    if (level) {
+        VTI_HIP(hipMemcpyAsync(W.sbtd.p, W.sbt.data(), sizeof(ShotB) * nw, hipMemcpyHostToDevice, st));
+        VTI_HIP(hipMemcpyAsync(W.tsh.p, W.tile_shot.data(), sizeof(int) * W.tile_shot.size(), hipMemcpyHostToDevice,
+                               st));
+        VTI_HIP(hipMemcpyAsync(W.tsht.p, W.tile_shot_t.data(), sizeof(int) * W.tile_shot_t.size(),
+                               hipMemcpyHostToDevice, st));
+        VTI_HIP(hipMemcpyAsync(W.recmap.p, hmap.data(), sizeof(int) * hmap.size(), hipMemcpyHostToDevice, st));
+    }
+    if (nrec && level) {
         VTI_HIP(hipMemcpyAsync(W.tsdd.p, tsd.data(), sizeof(int) * nrec, hipMemcpyHostToDevice, st));
         VTI_HIP(hipMemcpyAsync(W.fidxd.p, fidx.data(), sizeof(long long) * nrec, hipMemcpyHostToDevice, st));
         VTI_HIP(hipMemcpyAsync(W.tbd.p, tb.data(), sizeof(long long) * nrec, hipMemcpyHostToDevice, st));
     }
-    if (tr_total)
+    if (tr_total && a.grad)
         VTI_HIP(hipMemcpyAsync(W.obs.p, obs_h.data(), sizeof(float) * tr_total, hipMemcpyHostToDevice, st));
     VTI_HIP(hipStreamSynchronize(st));  // the host staging vectors end here
     return vti::kOk;
@@ -573,7 +631,8 @@ int enqueue_wave(BatchWave &W, BatchShared &S, const BatchArgs &a, const float *
     const int levels = a.levels, snap_fmt = a.snap_fmt;
     const bool half = a.half;
     DBuf<float> *P = W.P, *Q = W.Q, *G = W.G, *C = S.C;
-    for (int k = 0; k < 4; ++k) {
+    const bool res = a.res && !W.level;
+    for (int k = 0; k < 4 && !res; ++k) {
         zero_words(P[k].p, (size_t)f_total, st);
         zero_words(Q[k].p, (size_t)f_total, st);
     }
@@ -621,9 +680,14 @@ int enqueue_wave(BatchWave &W, BatchShared &S, const BatchArgs &a, const float *
     // ---- forward (objFuncGradient_f.cu:160-210 for every shot).  Buffers
     // ip/ic hold the previous and current levels; s0b/s1b are free.
     int ip = 1, ic = 0, s0b = 2, s1b = 3;
-    hipLaunchKernelGGL(set_src_b_kernel, dim3((nw + 63) / 64), dim3(64), 0, st, P[ic].p, Q[ic].p, sbd, nw,
-                       dt2 * wavelet[0]);
-    for (int it = 2; it < nt;) {
+    if (res) {
+        const int rc = W.res.forward(bg, dx2, dz2, dt2, C, t0d, W.tr.p, nt, false, sw, nnt - 1, st);
+        if (rc) return rc;
+    } else {
+        hipLaunchKernelGGL(set_src_b_kernel, dim3((nw + 63) / 64), dim3(64), 0, st, P[ic].p, Q[ic].p, sbd, nw,
+                           dt2 * wavelet[0]);
+    }
+    for (int it = res ? nt : 2; it < nt;) {
         if (levels == 2 && it + 1 < nt) {
             // levels it and it+1, reading levels it-1 and it
             const int sl1 = snap_slot(it - 1), sl2 = snap_slot(it);
@@ -651,9 +715,11 @@ int enqueue_wave(BatchWave &W, BatchShared &S, const BatchArgs &a, const float *
             it += 1;
         }
     }
-    hipLaunchKernelGGL(vti::dsnap2db_kernel, grid, block, 0, st, P[ic].p, Q[ic].p, sbd, tsh, bg, dx2, dz2, sw,
-                       nnt - 1);
-    pack(nnt - 1);
+    if (!res) {
+        hipLaunchKernelGGL(vti::dsnap2db_kernel, grid, block, 0, st, P[ic].p, Q[ic].p, sbd, tsh, bg, dx2, dz2, sw,
+                           nnt - 1);
+        pack(nnt - 1);
+    }
 
     // ---- residual and its partial sums (objFuncGradient_f.cu:214-219)
     if (per_shot_obj) {
@@ -674,7 +740,12 @@ int enqueue_wave(BatchWave &W, BatchShared &S, const BatchArgs &a, const float *
     }
 
     // ---- backward (objFuncGradient_f.cu:225-300 for every shot)
-    for (int k = 0; k < 4; ++k) {
+    if (res) {
+        const int rc = W.res.adjoint(bg, dx2, dz2, dt2, C, t0d, W.tr.p, sr, snap_fmt, a.nnt_data - 1, G[0].p, G[1].p,
+                                     G[2].p, st);
+        if (rc) return rc;
+    }
+    for (int k = 0; k < 4 && !res; ++k) {
         zero_words(P[k].p, (size_t)f_total, st);
         zero_words(Q[k].p, (size_t)f_total, st);
     }
@@ -682,10 +753,10 @@ int enqueue_wave(BatchWave &W, BatchShared &S, const BatchArgs &a, const float *
     ip = 1;
     s0b = 2;
     s1b = 3;
-    if (nrec)
+    if (nrec && !res)
         hipLaunchKernelGGL(inject_first_b_kernel, dim3(rb), dim3(256), 0, st, P[ic].p, Q[ic].p, W.tr.p, W.fidxd.p,
                            W.tbd.p, W.tsdd.p, nrec, a.nnt_data - 1, dt2);
-    {
+    if (!res) {
         float f = (float)((nt - 2.) / ratio);
         const int i1 = (int)f;
         f = f - i1;
@@ -698,20 +769,10 @@ int enqueue_wave(BatchWave &W, BatchShared &S, const BatchArgs &a, const float *
         else XCOR(3);
 #undef XCOR
     }
-    // trace rows and snapshot slots bracketing adjoint level it
-    auto level = [&](int it) {
-        vti::LevelB l;
-        float fr = (float)((it + 1.) / ratio);
-        l.row = (int)fr;
-        l.fr = fr - l.row;
-        float f = (float)it / ratio;
-        l.slot = (int)f;
-        l.f = f - l.slot;
-        return l;
-    };
+    auto level = [&](int it) { return adjoint_level(a, it); };
     int *recmap = W.recmap.p;
     float *tr = W.tr.p;
-    for (int it = nt - 3; it >= 0;) {
+    for (int it = res ? -1 : nt - 3; it >= 0;) {
         if (levels == 2 && it >= 1) {
             const vti::LevelB l1 = level(it), l2 = level(it - 1);
 #define BWD_T2(BYV, SFV)                                                                                         \
@@ -770,7 +831,7 @@ int enqueue_model_wave(BatchWave &W, BatchShared &S, const BatchArgs &a, const f
     const long long f_total = W.f_total;
     const float dx2 = a.dx2, dz2 = a.dz2, dt2 = a.dt2;
     DBuf<float> *P = W.P, *Q = W.Q, *C = S.C;
-    for (int k = 0; k < 4; ++k) {
+    for (int k = 0; k < 4 && !a.res; ++k) {
         zero_words(P[k].p, (size_t)f_total, st);
         zero_words(Q[k].p, (size_t)f_total, st);
     }
@@ -786,6 +847,8 @@ int enqueue_model_wave(BatchWave &W, BatchShared &S, const BatchArgs &a, const f
     const dim3 gridt((unsigned)W.tile_shot_t.size()), blockt(64, BYT);
     const int rb = (nrec + 255) / 256;
     const vti::SnapW sw{nullptr, nullptr};  // no snapshots (every slot argument is -1)
+    if (a.res)
+        return W.res.forward(bg, dx2, dz2, dt2, C, S.t0d.p, W.tr.p, nt, true, sw, -1, st);
     auto record = [&](int it, int buf) {
         if (it % ratio == 0 && nrec)
             hipLaunchKernelGGL(record_b_kernel, dim3(rb), dim3(256), 0, st, W.tr.p, P[buf].p, Q[buf].p, W.fidxd.p,
@@ -824,6 +887,10 @@ int enqueue_model_wave(BatchWave &W, BatchShared &S, const BatchArgs &a, const f
     return vti::kOk;
 }
 
+// Status of a wave that gave up its resident run (ResRun::aborted): its
+// results are void.
+constexpr int kGaveUp = 1;
+
 // the objective's share of a wave: the residual's partial sums, in order
 // Adds a wave's residual partial sums, shot by shot and block by block
 // (enqueue_wave with per_shot_obj), to obj[owner[s]] for batch shot s
@@ -831,6 +898,12 @@ int enqueue_model_wave(BatchWave &W, BatchShared &S, const BatchArgs &a, const f
 // the shots were split into waves.
 int wave_objective(const BatchWave &W, hipStream_t st, const int *owner, double *obj)
 {
+    bool gone = false;
+    if (W.res.active() && !W.level) {
+        const int rc = W.res.aborted(&gone, st);
+        if (rc) return rc;
+        if (gone) return kGaveUp;
+    }
     if (!W.tr_total) return vti::kOk;
     std::vector<double> hp(W.part.n);
     VTI_HIP(hipMemcpyAsync(hp.data(), W.part.p, sizeof(double) * hp.size(), hipMemcpyDeviceToHost, st));
@@ -870,7 +943,43 @@ std::vector<std::pair<int, int>> split_waves(const BatchArgs &a, int max_wave, l
     return w;
 }
 
-// Runs the waves of a batch, two in flight when there are several.  Wave k
+// Whether the call's shape arguments leave the launch form to the library:
+// the default, two levels per launch with 16-row tiles.
+bool res_wanted(const BatchArgs &a) { return a.levels == 2 && a.BYT == 16 && (a.snap_fmt == 0 || a.snap_fmt == 3); }
+
+// The waves of a call: resident ones (a.res is set) when every shot fits the
+// chip, as many consecutive shots as fit it together and at most max_res
+// (when > 0); else as split_waves with max_wave.
+std::vector<std::pair<int, int>> plan_waves(BatchArgs &a, int max_res, int max_wave, long long budget)
+{
+    a.res = false;
+    if (res_wanted(a)) {
+        std::vector<std::pair<int, int>> w;
+        std::vector<int> nnx;
+        for (int s0 = 0; s0 < a.ns;) {
+            long long used = 0;
+            int s1 = s0;
+            nnx.clear();
+            while (s1 < a.ns && (max_res <= 0 || s1 - s0 < max_res) &&
+                   (s1 == s0 || used + a.shot_bytes(s1) <= budget)) {
+                nnx.push_back(a.in[s1].nx + 2 * a.npad);
+                if (!vti::res_fits(nnx.data(), (int)nnx.size(), a.nnz, a.grad, a.snap_fmt)) break;
+                used += a.shot_bytes(s1++);
+            }
+            if (s1 == s0) break;
+            w.emplace_back(s0, s1);
+            s0 = s1;
+        }
+        if (!w.empty() && w.back().second == a.ns) {
+            a.res = true;
+            return w;
+        }
+    }
+    return split_waves(a, max_wave, budget);
+}
+
+// Runs the waves of a batch: one after the other, or (overlap) two in flight
+// when there are several.  Wave k
 // runs on stream k % 2 (st, or a second one made for the call) and starts its
 // forward pass when wave k-1's is done, so that it overlaps wave k-1's
 // adjoint (the forward is bound by VALU work, the adjoint waits on memory),
@@ -880,10 +989,19 @@ std::vector<std::pair<int, int>> split_waves(const BatchArgs &a, int max_wave, l
 // adds them.
 int run_waves(BatchShared &S, const BatchArgs &a, const std::vector<std::pair<int, int>> &waves,
               const float *data, const int *rloc, const float *wavelet, hipStream_t st, const int *owner,
-              double *obj)
+              double *obj, bool overlap)
 {
     int rc = vti::kOk;
     const size_t n = waves.size();
+    if (!overlap) {
+        for (size_t k = 0; k < n && !rc; ++k) {
+            BatchWave W;
+            rc = setup_wave(W, a, waves[k].first, waves[k].second, data, rloc, st);
+            if (!rc) rc = enqueue_wave(W, S, a, wavelet, st, true);
+            if (!rc) rc = wave_objective(W, st, owner, obj);
+        }
+        return rc;
+    }
     StreamPair sp;
     if (n > 1) rc = sp.init(st);
     auto stream_of = [&](size_t k) { return k % 2 ? sp.side : st; };
@@ -924,6 +1042,23 @@ int run_waves(BatchShared &S, const BatchArgs &a, const std::vector<std::pair<in
     return rc;  // (sp's destructor waits for both streams before it releases them)
 }
 
+// run_waves on the waves of plan_waves; should a resident wave give up, the
+// whole call again on the per-level kernels.  obj: nobj sums, S.A: the
+// gradient, both zero on entry.
+int run_planned(BatchShared &S, BatchArgs &a, int max_res, int max_wave, long long budget, const float *data,
+                const int *rloc, const float *wavelet, hipStream_t st, const int *owner, double *obj, int nobj,
+                bool overlap)
+{
+    a.wavelet = wavelet;
+    const auto waves = plan_waves(a, max_res, max_wave, budget);
+    const int rc = run_waves(S, a, waves, data, rloc, wavelet, st, owner, obj, overlap);
+    if (rc != kGaveUp) return rc;
+    a.res = false;
+    for (int k = 0; k < 3; ++k) zero_words(S.A[k].p, 2 * S.A[k].n, st);
+    std::fill(obj, obj + nobj, 0.0);
+    return run_waves(S, a, split_waves(a, max_wave, budget), data, rloc, wavelet, st, owner, obj, overlap);
+}
+
 // Shots per wave whose adjoint working set stays in the 256 MB Infinity
 // Cache: per shot and point 16 FP32 planes (four buffers of p and q, the
 // three gradients, the two snapshot slots a level reads, the receiver map),
@@ -955,7 +1090,8 @@ struct vti2d_batch_plan {
     BatchShared S;
     WavePool pool[2];
     std::vector<std::unique_ptr<BatchWave>> W;
-    std::vector<hipGraphExec_t> fwd, adj;
+    std::vector<hipGraphExec_t> fwd, adj;  // per-level waves only: a resident wave is a few launches
+    std::vector<float> w;
     hipStream_t side = nullptr;
     hipEvent_t ev_fwd[2] = {nullptr, nullptr}, ev_adj[2] = {nullptr, nullptr}, ev_join = nullptr;
 };
@@ -991,9 +1127,9 @@ int vti2d_objfunc_gradient_batch(vti_ctx *ctx, double *objfunc, double *gc11, do
     const size_t mfree = vti::device_free_bytes();
     const long long budget = ((long long)mfree - (long long)(2ULL << 30)) / 3;  // three waves set up at once
     VTI_CHECK(budget > a.shot_bytes(0), "not enough device memory for one shot");
-    const auto waves = split_waves(a, max_wave > 0 ? (max_wave + 1) / 2 : 0, budget);
+    const int mw = max_wave > 0 ? (max_wave + 1) / 2 : 0;
     double obj = 0.0;
-    rc = run_waves(S, a, waves, data, rloc, wavelet, st, nullptr, &obj);
+    rc = run_planned(S, a, mw, mw, budget, data, rloc, wavelet, st, nullptr, &obj, 1, true);
     if (rc) return rc;
     rc = download_gradient(S, a, gc11, gc13, gc33, st);
     if (rc) return rc;
@@ -1026,7 +1162,10 @@ int vti2d_batch_plan_create(vti_ctx *ctx, vti2d_batch_plan **plan, const float *
         // fits the largest wave that uses it, and each wave adds its own
         // tables and data
         const long long budget = (long long)vti::device_free_bytes() - (long long)(2ULL << 30);
-        for (const auto &w : split_waves(pl->a, max_wave > 0 ? (max_wave + 1) / 2 : 0, budget / 2)) {
+        const int mw = max_wave > 0 ? (max_wave + 1) / 2 : 0;
+        pl->w.assign(wavelet, wavelet + nt);
+        pl->a.wavelet = pl->w.data();
+        for (const auto &w : plan_waves(pl->a, mw, mw, budget / 2)) {
             pl->W.emplace_back(new BatchWave);
             size_wave(*pl->W.back(), pl->a, w.first, w.second, rloc);
             pool_fit(pl->pool[(pl->W.size() - 1) % 2], *pl->W.back(), pl->a);
@@ -1056,7 +1195,7 @@ int vti2d_batch_plan_create(vti_ctx *ctx, vti2d_batch_plan **plan, const float *
         if (rc) vti::set_error("vti2d_batch_plan_create: stream or event creation failed");
     }
     // each wave captured on its own, on one stream, as two graphs
-    for (size_t k = 0; k < pl->W.size() && !rc; ++k) {
+    for (size_t k = 0; k < pl->W.size() && !rc && !pl->a.res; ++k) {
         hipGraph_t g[2] = {nullptr, nullptr};
         hipError_t e = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal);
         bool capturing = e == hipSuccess;
@@ -1112,6 +1251,14 @@ int vti2d_batch_plan_run(vti2d_batch_plan *plan, double *objfunc, double *gc11, 
     }
     for (size_t k = 0; k < nw; ++k) {
         hipStream_t sk = k % 2 ? plan->side : st;
+        if (plan->a.res) {
+            WaveSync sync;
+            sync.acc_wait = k >= 1 ? plan->ev_adj[(k - 1) % 2] : nullptr;
+            sync.acc_done = nw > 1 ? plan->ev_adj[k % 2] : nullptr;
+            rc = enqueue_wave(*plan->W[k], plan->S, plan->a, plan->w.data(), sk, true, &sync);
+            if (rc) return rc;
+            continue;
+        }
         if (k >= 1) VTI_HIP(hipStreamWaitEvent(sk, plan->ev_fwd[(k - 1) % 2], 0));
         VTI_HIP(hipGraphLaunch(plan->fwd[k], sk));
         if (nw > 1) VTI_HIP(hipEventRecord(plan->ev_fwd[k % 2], sk));
@@ -1125,6 +1272,18 @@ int vti2d_batch_plan_run(vti2d_batch_plan *plan, double *objfunc, double *gc11, 
     double obj = 0.0;
     for (const auto &W : plan->W)
         if (!rc) rc = wave_objective(*W, st, nullptr, &obj);
+    if (rc == kGaveUp) {  // the whole run on the per-level kernels
+        obj = 0.0;
+        rc = vti::kOk;
+        VTI_HIP(hipStreamSynchronize(st));
+        for (int k = 0; k < 3; ++k) zero_words(plan->S.A[k].p, 2 * plan->S.A[k].n, st);
+        for (const auto &W : plan->W) {
+            W->level = true;
+            if (!rc) rc = enqueue_wave(*W, plan->S, plan->a, plan->w.data(), st, true);
+            if (!rc) rc = wave_objective(*W, st, nullptr, &obj);
+            W->level = false;
+        }
+    }
     if (!rc) rc = download_gradient(plan->S, plan->a, gc11, gc13, gc33, st);
     if (rc) return rc;
     *objfunc = 0.5 * obj;
@@ -1227,14 +1386,26 @@ int synth2d_batched(vti_ctx *ctx, float *out, const float *c11, const float *c13
     const float *cs[3] = {c11, c13, c33};
     for (int k = 0; k < 3; ++k)
         VTI_HIP(hipMemcpyAsync(S.C[k].p, cs[k], (size_t)nnx * nnz * 4, hipMemcpyDefault, st));
-    const std::vector<float> nodata((size_t)std::max<long long>((long long)nnt * (rl.size() / 2), 1), 0.f);
     const int cw = cache_wave(shots.data(), ns, npad, nz);
     const long long budget = (long long)vti::device_free_bytes() - (long long)(2ULL << 30);
-    for (const auto &wv : split_waves(a, cw, budget)) {
+    a.grad = false;
+    a.wavelet = wavelet;
+    auto waves = plan_waves(a, 0, cw, budget);
+    for (size_t k = 0; k < waves.size(); ++k) {
+        const auto wv = waves[k];
         BatchWave W;
-        rc = setup_wave(W, a, wv.first, wv.second, nodata.data(), rl.data(), st);
+        rc = setup_wave(W, a, wv.first, wv.second, nullptr, rl.data(), st);
         if (!rc) rc = enqueue_model_wave(W, S, a, wavelet, st);
         if (rc) return rc;
+        bool gone = false;
+        rc = W.res.aborted(&gone, st);
+        if (rc) return rc;
+        if (gone) {  // the whole call on the per-level kernels
+            a.res = false;
+            waves = split_waves(a, cw, budget);
+            k = (size_t)-1;
+            continue;
+        }
         std::vector<float> h((size_t)std::max<long long>(W.tr_total, 1));
         if (W.tr_total) VTI_HIP(hipMemcpyAsync(h.data(), W.tr.p, W.tr_total * 4, hipMemcpyDeviceToHost, st));
         VTI_HIP(hipStreamSynchronize(st));
@@ -1345,17 +1516,8 @@ int grad2d_merged(vti_ctx *ctx, const Grad2dPart *p, int n, const float *wavelet
         const int wave = max_wave > 0 ? std::min(max_wave, cw) : cw;
         const size_t mfree = vti::device_free_bytes();
         const long long budget = ((long long)mfree - (long long)(2ULL << 30)) / (overlap ? 3 : 1);
-        if (overlap)
-            rc = run_waves(S, a, split_waves(a, (wave + 1) / 2, budget), data.data(), rl.data(), wavelet, st,
-                           owner.data(), obj.data());
-        else
-            for (const auto &wv : split_waves(a, wave, budget)) {
-                BatchWave W;
-                rc = setup_wave(W, a, wv.first, wv.second, data.data(), rl.data(), st);
-                if (!rc) rc = enqueue_wave(W, S, a, wavelet, st, true);
-                if (!rc) rc = wave_objective(W, st, owner.data(), obj.data());
-                if (rc) break;
-            }
+        rc = run_planned(S, a, max_wave, overlap ? (wave + 1) / 2 : wave, budget, data.data(), rl.data(), wavelet, st,
+                         owner.data(), obj.data(), n, overlap);
         if (rc) return rc;
         // rounded to FP32 on the device
         const size_t g = (size_t)NNX * nnz;

@@ -308,7 +308,7 @@ __device__ __forceinline__ int slice_exp(unsigned mbits)
 // Round the staged slices of slot `slot` of every shot (blockIdx.y) to 16
 // bits (FP16 when bf16 == 0, else BF16; round to nearest even) and record
 // their scales.
-static __global__ void pack_snap_kernel(unsigned short *__restrict__ snap, float *__restrict__ scale,
+static __global__ __attribute__((unused)) void pack_snap_kernel(unsigned short *__restrict__ snap, float *__restrict__ scale,
                                         const float *__restrict__ stage, const unsigned *__restrict__ amax,
                                         const ShotB *__restrict__ shots, int nnz, int slot, int bf16)
 {
@@ -388,7 +388,7 @@ __device__ __forceinline__ void load_tiles_b(Tiles2 &t, const float *__restrict_
 // forwardC step of every shot with injectSource, abc and (slot >= 0) the D
 // snapshot of the level read (objFuncGradient_f.cu:160-210 per shot).  The
 // point's own operands are loaded with the tiles, before the barrier.
-static __global__ __launch_bounds__(64 * kBY2) void fwd2db_kernel(
+static __global__ __attribute__((unused)) __launch_bounds__(64 * kBY2) void fwd2db_kernel(
     float *__restrict__ P_n, float *__restrict__ Q_n, const float *__restrict__ P_c, const float *__restrict__ Q_c,
     const float *__restrict__ c11, const float *__restrict__ c13, const float *__restrict__ c33,
     const float *__restrict__ t0, const ShotB *__restrict__ shots, const int *__restrict__ tile_shot, BatchGeo bg,
@@ -443,7 +443,7 @@ static __global__ __launch_bounds__(64 * kBY2) void fwd2db_kernel(
 }
 
 // D of the last forward level of every shot into its snapshot slot
-static __global__ __launch_bounds__(64 * kBY2) void dsnap2db_kernel(const float *__restrict__ P,
+static __global__ __attribute__((unused)) __launch_bounds__(64 * kBY2) void dsnap2db_kernel(const float *__restrict__ P,
                                                                     const float *__restrict__ Q,
                                                                     const ShotB *__restrict__ shots,
                                                                     const int *__restrict__ tile_shot, BatchGeo bg,
