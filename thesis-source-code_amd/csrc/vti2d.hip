@@ -321,10 +321,13 @@ int vti2d_synthetic(vti_ctx *ctx, float *data, const float *c11, const float *c1
                     int nz, int nt, int npad, float dx, float dz, float dt, float rate, float ot)
 {
     // Several shots with the standard taper (and rate/dt rounding the same in
-    // float as in synthetic_f's double) run as one batch, bit for bit.
-    if (ctx && ns >= 2 && data && c11 && c13 && c33 && wavelet && dx > 0 && dz > 0 && dt > 0 &&
+    // float as in synthetic_f's double) run as one batch, bit for bit; so does one
+    // that fits the chip (136 x 120 points: 1.5 us a level resident, 4 us
+    // launch by launch).
+    if (ctx && ns >= 1 && data && c11 && c13 && c33 && wavelet && dx > 0 && dz > 0 && dt > 0 &&
         (int)(rate / dt + 0.5f) == (int)(rate / dt + 0.5) &&
-        vti::grad2d_batchable(sloc, ns, rloc, nr, taper, nx, nz, nt, npad, dt, rate, ot))
+        vti::grad2d_batchable(sloc, ns, rloc, nr, taper, nx, nz, nt, npad, dt, rate, ot) &&
+        (ns >= 2 || vti::res2d_fits(ctx, nx + 2 * npad, nz + 2 * npad, false)))
         return vti::synth2d_batched(ctx, data, c11, c13, c33, wavelet, sloc, ns, rloc, nr, nx, nz, nt, npad, dx, dz,
                                     dt, rate);
     Call2 c;
@@ -1142,10 +1145,13 @@ int vti2d_objfunc_gradient(vti_ctx *ctx, float *objfunc, float *gc11, float *gc1
     // launch for all of a wave's shots); each shot's gradient and objective
     // are the one-shot loop's, summed in the same order, so the result is the
     // same bit for bit.
-    // A context set to 16-bit snapshots sends single shots there too.
-    if (ctx && (ns >= 2 || (ns == 1 && ctx->snap_fmt != 0)) && objfunc && gc11 && gc13 && gc33 && data && c11 &&
+    // A context set to 16-bit snapshots sends single shots there too, and so
+    // does a shot that fits the chip (592 x 1104 points: 6.1 us for a forward and an
+    // adjoint level resident, 20.8 us launch by launch).
+    if (ctx && ns >= 1 && objfunc && gc11 && gc13 && gc33 && data && c11 &&
         c13 && c33 && wavelet && dx > 0 && dz > 0 &&
-        vti::grad2d_batchable(sloc, ns, rloc, nr, taper, nx, nz, nt, npad, dt, rate, ot)) {
+        vti::grad2d_batchable(sloc, ns, rloc, nr, taper, nx, nz, nt, npad, dt, rate, ot) &&
+        (ns >= 2 || ctx->snap_fmt != 0 || vti::res2d_fits(ctx, nx + 2 * npad, nz + 2 * npad, true))) {
         vti::Grad2dPart part;
         part.c[0] = c11;
         part.c[1] = c13;

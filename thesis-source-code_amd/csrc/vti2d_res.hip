@@ -5,6 +5,7 @@
 #include <mutex>
 #include <type_traits>
 
+#include "vti_ctx.h"
 #include "vti_internal.h"
 
 namespace vti {
@@ -134,6 +135,15 @@ int res_rows(const int *nnx, int ns, int nnz, bool adjoint, int snap_fmt)
 bool res_fits(const int *nnx, int ns, int nnz, bool grad, int snap_fmt)
 {
     return res_rows(nnx, ns, nnz, false, snap_fmt) && (!grad || res_rows(nnx, ns, nnz, true, snap_fmt));
+}
+
+bool res2d_fits(vti_ctx *ctx, int nnx, int nnz, bool grad)
+{
+    if (hipSetDevice(ctx->device) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return res_fits(&nnx, 1, nnz, grad, 0);
 }
 
 namespace {

@@ -78,6 +78,10 @@ long long grad2d_merged_bytes(const Grad2dPart *p, int n, int nz, int nt, int np
 int grad2d_merged(vti_ctx *ctx, const Grad2dPart *p, int n, const float *wavelet, int nz, int nt, int npad,
                   float dx, float dz, float dt, float rate, int max_wave, int snap_fmt, bool overlap = false);
 
+// whether a shot of nnx x nnz points runs resident (vti2d_res.h) on ctx's
+// device: its forward pass, and with grad its adjoint
+bool res2d_fits(vti_ctx *ctx, int nnx, int nnz, bool grad);
+
 int dmalloc(void **p, size_t bytes, hipStream_t s);
 // free device memory of the current device, counting the large blocks
 // dmalloc keeps for reuse
