@@ -6,7 +6,7 @@ and through the fallback for a grid that does not fit the chip."""
 import numpy as np
 import pytest
 
-from common2d import layered2d
+from common2d import args2d, layered2d, problem2d
 from common3d import cij_from, ricker
 
 pytestmark = pytest.mark.gpu
@@ -58,3 +58,21 @@ def test_grid_beyond_the_chip(vti, ctx):
     f0, g0 = vti.objfunc_gradient2d_batch(ctx, data, *c, w, shots, rloc, *rest, levels=1)
     f1, g1 = vti.objfunc_gradient2d_batch(ctx, data, *c, w, shots, rloc, *rest)
     assert f0 == f1 and np.array_equal(g0, g1)
+
+
+@pytest.mark.parametrize("nx,nz,npad,nt", [(2, 5, 4, 21), (64, 12, 4, 61), (65, 17, 4, 61), (131, 97, 5, 81),
+                                           (300, 130, 12, 41)])
+def test_resident_product_and_image_vs_oracle(vti, orc, ctx, nx, nz, npad, nt):
+    """The Gauss-Newton product and the RTM image of a shot that fits the chip
+    equal the oracle's FP32 restatement bit for bit at the edges of the tiles."""
+    P = problem2d(vti, nx=nx, nz=nz, npad=npad, nt=nt, ns=1)
+    print("resident product and image", nx, nz, npad, nt, flush=True)
+    dc = [(1e-2 * (a - b)).astype(np.float32) for a, b in zip(P["ctrue"], P["c"])]
+    dc[0][:, ::3] += np.float32(1e3)
+    a = args2d(P)
+    h = vti.gn_hessian2d(ctx, *P["c"], *dc, P["w"], P["sloc"], P["rloc"], P["taper"], *a)
+    ho = orc.fg2d(orc.F32, True, None, *P["c"], dc, P["w"], P["sloc"], P["rloc"], P["taper"], *a)[1]
+    assert np.array_equal(h, ho)
+    data = (1e-7 * np.random.default_rng(3).standard_normal(((nt - 1) // 4 + 1, P["nr"]))).astype(np.float32)
+    img = vti.rtm2d(ctx, data, *P["c"], P["w"], P["sloc"], P["rloc"], P["taper"], *a)
+    assert np.array_equal(img, orc.rtm2d(orc.F32, data, *P["c"], P["w"], P["sloc"], P["rloc"], P["taper"], *a))

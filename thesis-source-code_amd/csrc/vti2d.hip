@@ -17,6 +17,7 @@
 #include "vti2d_kernels.h"
 #include "vti_dbuf.h"
 #include "vti_ctx.h"
+#include "vti_host.h"
 #include "vti_internal.h"
 
 using vti::DBuf;
@@ -298,6 +299,21 @@ int load_model(const Call2 &c, Fields2 &F, const float *c11, const float *c13, c
     if (!rc) rc = upload(c, F.c33.p, c33, n * 4);
     if (!rc) rc = upload(c, F.taper.p, taper, n * 4);
     return rc;
+}
+
+// whether taper is init_abc's, bit for bit
+bool standard_taper(const Call2 &c, const float *taper)
+{
+    std::vector<float> t((size_t)c.nnxz);
+    vti::init_taper2d(t.data(), c.nx, c.nz, c.npad);
+    return std::memcmp(t.data(), taper, t.size() * sizeof(float)) == 0;
+}
+
+// a shot as the resident passes take it
+vti::Res2dShot res_shot(const Call2 &c, const Shot2 &s, const int *rloc, const Fields2 &F, float *tr)
+{
+    return vti::Res2dShot{c.ctx, c.g.nnx, c.g.nnz, c.npad, c.nt, c.ratio, s.nri, s.src, rloc + 2 * (size_t)s.r0,
+                          c.dx2, c.dz2, c.dt2, {F.c11.p, F.c13.p, F.c33.p}, tr};
 }
 
 int zero2(const Call2 &c, DBuf<float> *a, DBuf<float> *b)
@@ -646,6 +662,9 @@ int rtm2d(vti_ctx *ctx, int nhx, float *image, const float *data, const float *c
     if (!rc) rc = recmap.alloc(n, st);
     if (!rc) rc = dipmap.alloc(n, st);
     if (rc) return rc;
+    // resident passes (vti2d_res1.hip) where the shot fits the chip: 456 x 732
+    // points, 2.4 us a level against 4.8-5.5 launch by launch
+    const bool std_taper = standard_taper(c, taper);
     const dim3 rows((c.g.nnx - 8 + 255) / 256, c.g.nnz - 8);
     const int xlo = odcig ? std::max(4, nhx) : 4;
     const dim3 xrows((std::max(1, c.g.nnx - 2 * xlo) + 255) / 256, c.g.nnz - 8);
@@ -685,13 +704,17 @@ int rtm2d(vti_ctx *ctx, int nhx, float *image, const float *data, const float *c
         VTI_HIP(hipMemsetAsync(img.p, 0, n * nh * 4, st));
 
         // ---- source side (rtm_f.cu:110-150)
-        rc = zero2(c, F.p, F.q);
+        const vti::Res2dShot rs = res_shot(c, s, rloc, F, tr.p);
+        bool by_level = !(std_taper && vti::res2d_fits_slices(rs));
+        if (!by_level) rc = vti::res2d_slices(rs, wavelet, !odcig, slices.p, &by_level);
+        if (!rc) rc = zero2(c, F.p, F.q);
         if (rc) return rc;
-        hipLaunchKernelGGL(dipole_level1_kernel, dim3(1), dim3(1), 0, st, F.p[0].p, F.q[0].p, F.taper.p, s.src,
-                           c.g.nnx, c.dt2 * wavelet[0]);
-        if (c.ratio == 1)
+        if (by_level)
+            hipLaunchKernelGGL(dipole_level1_kernel, dim3(1), dim3(1), 0, st, F.p[0].p, F.q[0].p, F.taper.p, s.src,
+                               c.g.nnx, c.dt2 * wavelet[0]);
+        if (by_level && c.ratio == 1)
             hipLaunchKernelGGL(slice2d_kernel, rows, dim3(256), 0, st, slices.p + n, F.p[0].p, F.q[0].p, c.g);
-        for (int it = 2; it < nt; ++it) {
+        for (int it = 2; by_level && it < nt; ++it) {
             // odcig_f.cu:123 injects wavelet[it-1] without the dt2 of its first level
             const float sv = odcig ? wavelet[it - 1] : c.dt2 * wavelet[it - 1];
             hipLaunchKernelGGL((vti::fwd2d_kernel<false>), c.grid, c.block, 0, st, F.p[1].p, F.q[1].p, F.p[0].p,
@@ -707,13 +730,18 @@ int rtm2d(vti_ctx *ctx, int nhx, float *image, const float *data, const float *c
         VTI_HIP(hipGetLastError());
 
         // ---- receiver side and imaging (rtm_f.cu:152-216)
-        rc = zero2(c, F.p, F.q);
+        by_level = odcig || !(std_taper && vti::res2d_fits_image(rs));
+        if (!by_level) {
+            rc = vti::res2d_image(rs, c.ntNeg, c.nnt_data - 1, slices.p, img.p, &by_level);
+            if (!rc && by_level) VTI_HIP(hipMemsetAsync(img.p, 0, n * nh * 4, st));
+        }
+        if (!rc) rc = zero2(c, F.p, F.q);
         if (rc) return rc;
-        if (s.nri)
+        if (by_level && s.nri)
             hipLaunchKernelGGL(dipole_first_kernel, dim3((s.nri + 255) / 256), dim3(256), 0, st, F.p[0].p, F.q[0].p,
                                F.taper.p, idx.p, tr.p + (size_t)(c.nnt_data - 1) * s.nri, s.nri, c.g.nnx, c.dt2);
         auto slot = [&](int k) { return slices.p + (size_t)k * n; };
-        {
+        if (by_level) {
             float f = (float)((nt - 2.) / c.ratio);
             const int i1 = (int)f;
             f = f - i1;
@@ -724,7 +752,7 @@ int rtm2d(vti_ctx *ctx, int nhx, float *image, const float *data, const float *c
                 hipLaunchKernelGGL(image2d_kernel, rows, dim3(256), 0, st, img.p, F.p[0].p, F.q[0].p, slot(i1),
                                    slot(i1 + 1), f, c.g);
         }
-        for (int it = nt - 3; it >= 0; --it) {
+        for (int it = nt - 3; by_level && it >= 0; --it) {
             // the data rows bracketing the level: row i1 and row i1+1 (zero past the last)
             int inj = 0, ir1 = 0;
             float fr = 0.f;
@@ -810,6 +838,11 @@ int fg2d(vti_ctx *ctx, bool born, float *objfunc, float *gc11, float *gc13, floa
     if (rc) return rc;
     auto snap_p = [&](int k) { return snap.p + (size_t)k * 2 * n; };
     auto snap_q = [&](int k) { return snap.p + (size_t)k * 2 * n + n; };
+    // the Gauss-Newton product's passes run resident (vti2d_res1.hip) where
+    // the shot fits the chip: 381 x 497 points, 2.7 us a level against 5.4-6.7
+    // launch by launch.  (The gradient's shots have come here because they do
+    // not.)
+    const bool std_taper = born && standard_taper(c, taper);
     double obj = 0.0;
     std::vector<int> hmap(n, -1);
     for (int is = 0; is < ns; ++is) {
@@ -834,12 +867,22 @@ int fg2d(vti_ctx *ctx, bool born, float *objfunc, float *gc11, float *gc13, floa
         if (!rc) rc = upload(c, recmap.p, hmap.data(), n * sizeof(int));
         if (rc) return rc;
 
+        const vti::Res2dShot rs = res_shot(c, s, rloc, F, bg.p);
+        bool by_level = !(std_taper && vti::res2d_fits_gn(rs));
+        if (!by_level) {
+            const float *dcp[3] = {dc[0].p, dc[1].p, dc[2].p};
+            rc = vti::res2d_gn(rs, dcp, wavelet, snap.p, acc[0].p, acc[1].p, acc[2].p, &by_level);
+            for (int k = 0; k < 3 && !rc && by_level; ++k) VTI_HIP(hipMemsetAsync(acc[k].p, 0, n * 4, st));
+            if (rc) return rc;
+        }
+
         // ---- forward (objFuncGradient_f.cu:160-210 / hessian_f.cu:735-806)
         rc = zero2(c, F.p, F.q);
         if (!rc && born) rc = zero2(c, B.p, B.q);
         if (rc) return rc;
-        hipLaunchKernelGGL(set2_kernel, dim3(1), dim3(1), 0, st, F.p[0].p, F.q[0].p, s.src, c.dt2 * wavelet[0]);
-        for (int it = 2; it < nt; ++it) {
+        if (by_level)
+            hipLaunchKernelGGL(set2_kernel, dim3(1), dim3(1), 0, st, F.p[0].p, F.q[0].p, s.src, c.dt2 * wavelet[0]);
+        for (int it = 2; by_level && it < nt; ++it) {
             // the step computing level it reads level it-1: snapshot its D when due
             const int lc = it - 1;
             float *sp = nullptr, *sq = nullptr;
@@ -869,8 +912,9 @@ int fg2d(vti_ctx *ctx, bool born, float *objfunc, float *gc11, float *gc13, floa
                                    bg.p + (size_t)(it / c.ratio) * s.nri, rp->p, rq->p, idx.p, s.nri);
             }
         }
-        hipLaunchKernelGGL(vti::dsnap2d_kernel, c.grid, c.block, 0, st, F.p[0].p, F.q[0].p, c.g, c.dx2, c.dz2,
-                           snap_p(c.nnt - 1), snap_q(c.nnt - 1));
+        if (by_level)
+            hipLaunchKernelGGL(vti::dsnap2d_kernel, c.grid, c.block, 0, st, F.p[0].p, F.q[0].p, c.g, c.dx2, c.dz2,
+                               snap_p(c.nnt - 1), snap_q(c.nnt - 1));
         VTI_HIP(hipGetLastError());
 
         // ---- residual and objective (objFuncGradient_f.cu:214-219)
@@ -892,10 +936,10 @@ int fg2d(vti_ctx *ctx, bool born, float *objfunc, float *gc11, float *gc13, floa
         // ---- backward (objFuncGradient_f.cu:225-300 / hessian_f.cu:834-900)
         rc = zero2(c, F.p, F.q);
         if (rc) return rc;
-        if (s.nri)
+        if (by_level && s.nri)
             hipLaunchKernelGGL(inject2d_kernel, dim3((s.nri + 255) / 256), dim3(256), 0, st, F.p[0].p, F.q[0].p,
                                idx.p, bg.p + (size_t)(c.nnt_data - 1) * s.nri, zrow.p, 0.f, s.nri, c.dt2);
-        {
+        if (by_level) {
             float f = (float)((nt - 2.) / c.ratio);
             const int i1 = (int)f;
             f = f - i1;
@@ -903,7 +947,7 @@ int fg2d(vti_ctx *ctx, bool born, float *objfunc, float *gc11, float *gc13, floa
                                F.p[0].p, F.q[0].p, snap_p(i1), snap_q(i1), snap_p(i1 + 1), snap_q(i1 + 1), f,
                                acc[0].p, acc[1].p, acc[2].p, c.g);
         }
-        for (int it = nt - 3; it >= 0; --it) {
+        for (int it = nt - 3; by_level && it >= 0; --it) {
             float fr = (float)((it + 1.) / c.ratio);
             const int ir1 = (int)fr;
             fr = fr - ir1;

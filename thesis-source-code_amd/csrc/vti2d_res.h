@@ -2,6 +2,9 @@
 // tables and the launches.
 #pragma once
 
+#include <algorithm>
+#include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "vti2d_res_kernels.h"
@@ -21,12 +24,122 @@ struct ResTiles {
     DBuf<u64> halo;
 };
 
+// Workgroups of a kernel that a CU holds for certain.  Other kernels may
+// come and go while a launch's workgroups are placed, so registers and LDS can
+// be left in pieces; with k-1 workgroups anywhere in a CU, the largest of the
+// k gaps holds another one if each takes at most 1/(2k-1) of it.  (Filling the
+// CUs to the last register has left workgroups outside, and the others
+// waiting for them.)  A workgroup has one wavefront on each SIMD.
+template <class F>
+int res_per_cu(F *kernel)
+{
+    hipFuncAttributes fa;
+    if (hipFuncGetAttributes(&fa, reinterpret_cast<const void *>(kernel)) != hipSuccess) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    if (fa.localSizeBytes) return 0;  // scratch would be another thing to wait for
+    const int regs = std::max(1, (fa.numRegs + 7) / 8 * 8), lds = std::max<int>(1, (int)fa.sharedSizeBytes);
+    int k = 0;
+    while (regs * (2 * k + 1) <= 512 && lds * (2 * k + 1) <= 160 * 1024 && k < 8) ++k;
+    return k;
+}
+
+// f(integral constant NR) for one of the built row counts
+template <class F>
+auto with_rows(int nr, F &&f)
+{
+    switch (nr) {
+    case 1: return f(std::integral_constant<int, 1>());
+    case 2: return f(std::integral_constant<int, 2>());
+    case 3: return f(std::integral_constant<int, 3>());
+    case 4: return f(std::integral_constant<int, 4>());
+    default: return f(std::integral_constant<int, 6>());
+    }
+}
+
+// The row count of the least cost(rows, tiles per CU) among those whose tiles
+// of these shots are all on the current device at once, cap(rows) on a CU;
+// 0 when there is none.
+template <class Cap, class Cost>
+int res_best_rows(const int *nnx, int ns, int nnz, Cap &&cap, Cost &&cost)
+{
+    int dev = 0, cus = 0, best = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    double least = 0;
+    for (int nr : {1, 2, 3, 4, 6}) {
+        const int th = kResNW * nr;
+        long long tiles = 0;
+        for (int s = 0; s < ns; ++s) tiles += (long long)((nnx[s] - 8 + 63) / 64) * ((nnz - 8 + th - 1) / th);
+        if (tiles > (long long)cus * cap(nr)) continue;
+        const double c = cost(nr, (double)tiles / cus);
+        if (best && c >= least) continue;
+        best = nr;
+        least = c;
+    }
+    return best;
+}
+
+// Resident launches of one device follow one another, whatever their
+// streams: two that each hold part of the chip would wait for their missing
+// workgroups for ever.  The mutex covers the enqueueing only.
+struct ResGate {
+    std::mutex mu;
+    hipEvent_t done = nullptr;
+};
+ResGate &res_gate(int dev);
+void res_clear(const DBuf<u64> &halo, hipStream_t st);
+// clears the strips, then launch(), behind the device's last resident launch
+template <class Launch>
+int res_launch(const DBuf<u64> &halo, hipStream_t st, Launch &&launch)
+{
+    int dev = 0;
+    VTI_HIP(hipGetDevice(&dev));
+    ResGate &g = res_gate(dev);
+    std::lock_guard<std::mutex> lk(g.mu);
+    if (g.done)
+        VTI_HIP(hipStreamWaitEvent(st, g.done, 0));
+    else
+        VTI_HIP(hipEventCreateWithFlags(&g.done, hipEventDisableTiming));
+    res_clear(halo, st);
+    launch();
+    VTI_HIP(hipGetLastError());
+    VTI_HIP(hipEventRecord(g.done, st));
+    return kOk;
+}
+
 // The rows per wavefront with which shots of these padded widths (nnz rows
 // each) are all on the current device at once in a pass (adjoint or forward;
 // snap_fmt 0 or 3), the fastest of them; 0 when there is none.
 int res_rows(const int *nnx, int ns, int nnz, bool adjoint, int snap_fmt);
 // whether the shots fit in the forward pass and, with grad, in the adjoint
 bool res_fits(const int *nnx, int ns, int nnz, bool grad, int snap_fmt);
+
+// Tables of the shots base (all fields but tile0/ntx as the caller keeps
+// them) in tiles of nr rows a wavefront, and the receivers of each: rxz[2 r0[j]
+// ..] holds shot j's (ix, iz).  Points outside the interior, where the fields
+// stay 0, are left out.  nf: field pairs exchanged; dipole: the point below
+// each receiver is its negative pole.  The host tables stay in place until the
+// stream has read them.
+int res_setup(ResTiles &t, int nr, const std::vector<ShotB> &base, int nnz, const int *rxz, const int *r0,
+              hipStream_t st, int nf = 1, bool dipole = false);
+ResArgs res_args(const ResTiles &t, int *abort, const BatchGeo &bg, float dx2, float dz2, float dt2, const float *c11,
+                 const float *c13, const float *c33, const float *t0, float *tr);
+// after the stream is idle: whether a wait ran out
+int res_gave_up(const DBuf<int> &abort, bool *yes, hipStream_t st);
+
+template <class T>
+int res_upload(DBuf<T> &d, const std::vector<T> &h, hipStream_t st)
+{
+    const int rc = d.alloc(h.size(), st, false);
+    if (rc) return rc;
+    if (!h.empty()) VTI_HIP(hipMemcpyAsync(d.p, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice, st));
+    return kOk;
+}
 
 // One set of shots run resident.
 struct ResRun {
@@ -38,10 +151,7 @@ struct ResRun {
     DBuf<LevelB> lbd;
 
     bool active() const { return f.nr > 0; }
-    // Tables for the shots base (all fields but tile0/ntx as the caller keeps
-    // them) and the receivers of each: rxz[2 r0[j] ..] holds shot j's (ix, iz).
-    // Points outside the interior, where the fields stay 0, are left out.
-    // The host tables stay in place until the stream has read them.
+    // the tables of both passes (res_setup)
     int setup(const std::vector<ShotB> &base, int nnz, int snap_fmt, const int *rxz, const int *r0, hipStream_t st);
     int forward(const BatchGeo &bg, float dx2, float dz2, float dt2, const DBuf<float> *c, const float *t0, float *tr,
                 int nt, bool taper_first, const SnapW &sw, int last_snap, hipStream_t st);

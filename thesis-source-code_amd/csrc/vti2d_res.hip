@@ -2,8 +2,6 @@
 #include "vti2d_res.h"
 
 #include <algorithm>
-#include <mutex>
-#include <type_traits>
 
 #include "vti_ctx.h"
 #include "vti_internal.h"
@@ -12,27 +10,6 @@ namespace vti {
 
 namespace {
 
-// Workgroups of a kernel that a CU holds for certain.  Other kernels may
-// come and go while a launch's workgroups are placed, so registers and LDS can
-// be left in pieces; with k-1 workgroups anywhere in a CU, the largest of the
-// k gaps holds another one if each takes at most 1/(2k-1) of it.  (Filling the
-// CUs to the last register has left workgroups outside, and the others
-// waiting for them.)  A workgroup has one wavefront on each SIMD.
-template <class F>
-int res_per_cu(F *kernel)
-{
-    hipFuncAttributes fa;
-    if (hipFuncGetAttributes(&fa, reinterpret_cast<const void *>(kernel)) != hipSuccess) {
-        (void)hipGetLastError();
-        return 0;
-    }
-    if (fa.localSizeBytes) return 0;  // scratch would be another thing to wait for
-    const int regs = std::max(1, (fa.numRegs + 7) / 8 * 8), lds = std::max<int>(1, (int)fa.sharedSizeBytes);
-    int k = 0;
-    while (regs * (2 * k + 1) <= 512 && lds * (2 * k + 1) <= 160 * 1024 && k < 8) ++k;
-    return k;
-}
-
 template <int NR>
 int per_cu(bool adjoint, int snap_fmt)
 {
@@ -40,96 +17,35 @@ int per_cu(bool adjoint, int snap_fmt)
     return snap_fmt == 3 ? res_per_cu(bwd2d_res_kernel<NR, 3>) : res_per_cu(bwd2d_res_kernel<NR, 0>);
 }
 
-// f(integral constant NR) for one of the built row counts
-template <class F>
-auto with_rows(int nr, F &&f)
-{
-    switch (nr) {
-    case 1: return f(std::integral_constant<int, 1>());
-    case 2: return f(std::integral_constant<int, 2>());
-    case 3: return f(std::integral_constant<int, 3>());
-    case 4: return f(std::integral_constant<int, 4>());
-    default: return f(std::integral_constant<int, 6>());
-    }
-}
-
-// Resident launches of one device follow one another, whatever their
-// streams: two that each hold part of the chip would wait for their missing
-// workgroups for ever.  The mutex covers the enqueueing only.
-struct Gate {
-    std::mutex mu;
-    hipEvent_t done = nullptr;
-};
-Gate &gate(int dev)
-{
-    static Gate *g = new Gate[64];  // outlives static destructors
-    return g[dev & 63];
-}
-
-template <class Launch>
-int gated(hipStream_t st, Launch &&launch)
-{
-    int dev = 0;
-    VTI_HIP(hipGetDevice(&dev));
-    Gate &g = gate(dev);
-    std::lock_guard<std::mutex> lk(g.mu);
-    if (g.done)
-        VTI_HIP(hipStreamWaitEvent(st, g.done, 0));
-    else
-        VTI_HIP(hipEventCreateWithFlags(&g.done, hipEventDisableTiming));
-    launch();
-    VTI_HIP(hipGetLastError());
-    VTI_HIP(hipEventRecord(g.done, st));
-    return kOk;
-}
-
 __global__ void zero64_kernel(u64 *__restrict__ p, long long n)
 {
     for (long long k = blockIdx.x * (long long)blockDim.x + threadIdx.x; k < n; k += (long long)gridDim.x * blockDim.x)
         p[k] = 0;
 }
-void clear_halo(const DBuf<u64> &h, hipStream_t st)
+}  // namespace
+
+ResGate &res_gate(int dev)
+{
+    static ResGate *g = new ResGate[64];  // outlives static destructors
+    return g[dev & 63];
+}
+
+void res_clear(const DBuf<u64> &h, hipStream_t st)
 {
     const unsigned nb = (unsigned)std::max<size_t>(1, std::min<size_t>((h.n + 255) / 256, 4096));
     hipLaunchKernelGGL(zero64_kernel, dim3(nb), dim3(256), 0, st, h.p, (long long)h.n);
 }
 
-template <class T>
-int upload(DBuf<T> &d, const std::vector<T> &h, hipStream_t st)
-{
-    const int rc = d.alloc(h.size(), st, false);
-    if (rc) return rc;
-    if (!h.empty()) VTI_HIP(hipMemcpyAsync(d.p, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice, st));
-    return kOk;
-}
-
-}  // namespace
-
 int res_rows(const int *nnx, int ns, int nnz, bool adjoint, int snap_fmt)
 {
-    int dev = 0, cus = 0, best = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
-        (void)hipGetLastError();
-        return 0;
-    }
-    double cost = 0;
-    for (int nr : {1, 2, 3, 4, 6}) {
-        const int th = kResNW * nr;
-        long long tiles = 0;
-        for (int s = 0; s < ns; ++s) tiles += (long long)((nnx[s] - 8 + 63) / 64) * ((nnz - 8 + th - 1) / th);
-        const int cap = with_rows(nr, [&](auto n) { return per_cu<n.value>(adjoint, snap_fmt); });
-        if (tiles > (long long)cus * cap) continue;
-        // us a level takes, from runs of 10 to 984 tiles: the exchange, a
-        // wavefront's rows one after the other, and the tiles' traffic
-        // (forward 1.50 at 1 row and 56 tiles, 2.81 at 4 and 666, 3.08 at 6 and
-        // 450; adjoint 1.64 at 1 and 56, 2.59 at 4 and 407, 3.31 at 6 and 450)
-        const double c = adjoint ? 1.3 + 0.28 * nr + 0.2 * (double)tiles / cus : 1.15 + 0.22 * nr + 0.38 * (double)tiles / cus;
-        if (best && c >= cost) continue;
-        best = nr;
-        cost = c;
-    }
-    return best;
+    // us a level takes, from runs of 10 to 984 tiles: the exchange, a
+    // wavefront's rows one after the other, and the tiles' traffic
+    // (forward 1.50 at 1 row and 56 tiles, 2.81 at 4 and 666, 3.08 at 6 and
+    // 450; adjoint 1.64 at 1 and 56, 2.59 at 4 and 407, 3.31 at 6 and 450)
+    return res_best_rows(
+        nnx, ns, nnz,
+        [&](int nr) { return with_rows(nr, [&](auto n) { return per_cu<n.value>(adjoint, snap_fmt); }); },
+        [&](int nr, double t) { return adjoint ? 1.3 + 0.28 * nr + 0.2 * t : 1.15 + 0.22 * nr + 0.38 * t; });
 }
 
 bool res_fits(const int *nnx, int ns, int nnz, bool grad, int snap_fmt)
@@ -146,10 +62,8 @@ bool res2d_fits(vti_ctx *ctx, int nnx, int nnz, bool grad)
     return res_fits(&nnx, 1, nnz, grad, 0);
 }
 
-namespace {
-
-int setup_tiles(ResTiles &t, int nr, const std::vector<ShotB> &base, int nnz, const int *rxz, const int *r0,
-                hipStream_t st)
+int res_setup(ResTiles &t, int nr, const std::vector<ShotB> &base, int nnz, const int *rxz, const int *r0,
+              hipStream_t st, int nf, bool dipole)
 {
     VTI_CHECK(nr > 0, "the shots do not fit the chip");
     const int th = kResNW * nr, ns = (int)base.size();
@@ -169,13 +83,14 @@ int setup_tiles(ResTiles &t, int nr, const std::vector<ShotB> &base, int nnz, co
     };
     std::vector<Item> items;
     for (int j = 0; j < ns; ++j)
-        for (int k = 0; k < t.sb[j].nr; ++k) {
-            const int x = rxz[2 * ((size_t)r0[j] + k)] - 4, z = rxz[2 * ((size_t)r0[j] + k) + 1] - 4;
-            if (x < 0 || x >= t.sb[j].nnx - 8 || z < 0 || z >= nnz - 8) continue;
-            const int row = z % th, col = x & 63;
-            items.push_back({t.sb[j].tile0 + (x >> 6) + (z / th) * t.sb[j].ntx, ((row / nr) * 64 + col) * nr + row % nr,
-                             ResRec{row * 64 + col, k}});
-        }
+        for (int k = 0; k < t.sb[j].nr; ++k)
+            for (int pole = 0; pole < (dipole ? 2 : 1); ++pole) {
+                const int x = rxz[2 * ((size_t)r0[j] + k)] - 4, z = rxz[2 * ((size_t)r0[j] + k) + 1] - 4 + pole;
+                if (x < 0 || x >= t.sb[j].nnx - 8 || z < 0 || z >= nnz - 8) continue;
+                const int row = z % th, col = x & 63;
+                items.push_back({t.sb[j].tile0 + (x >> 6) + (z / th) * t.sb[j].ntx,
+                                 ((row / nr) * 64 + col) * nr + row % nr, ResRec{row * 64 + col, pole ? ~k : k}});
+            }
     std::stable_sort(items.begin(), items.end(),
                      [](const Item &a, const Item &b) { return a.tile != b.tile ? a.tile < b.tile : a.key < b.key; });
     t.rec_at.assign(t.ntiles + 1, 0);
@@ -185,16 +100,16 @@ int setup_tiles(ResTiles &t, int nr, const std::vector<ShotB> &base, int nnz, co
         t.rec.push_back(i.r);
     }
     for (int k = 0; k < t.ntiles; ++k) t.rec_at[k + 1] += t.rec_at[k];
-    int rc = upload(t.sbd, t.sb, st);
-    if (!rc) rc = upload(t.tsd, t.tile_shot, st);
-    if (!rc) rc = upload(t.rad, t.rec_at, st);
-    if (!rc) rc = upload(t.recd, t.rec, st);
-    if (!rc) rc = t.halo.alloc((size_t)t.ntiles * 2 * (8 * th + 512), st, false);
+    int rc = res_upload(t.sbd, t.sb, st);
+    if (!rc) rc = res_upload(t.tsd, t.tile_shot, st);
+    if (!rc) rc = res_upload(t.rad, t.rec_at, st);
+    if (!rc) rc = res_upload(t.recd, t.rec, st);
+    if (!rc) rc = t.halo.alloc((size_t)t.ntiles * 2 * nf * (8 * th + 512), st, false);
     return rc;
 }
 
-ResArgs res_args(const ResTiles &t, int *abort, const BatchGeo &bg, float dx2, float dz2, float dt2,
-                 const DBuf<float> *c, const float *t0, float *tr)
+ResArgs res_args(const ResTiles &t, int *abort, const BatchGeo &bg, float dx2, float dz2, float dt2, const float *c11,
+                 const float *c13, const float *c33, const float *t0, float *tr)
 {
     ResArgs a{};
     a.shots = t.sbd.p;
@@ -207,26 +122,24 @@ ResArgs res_args(const ResTiles &t, int *abort, const BatchGeo &bg, float dx2, f
     a.dt2 = dt2;
     a.halo = t.halo.p;
     a.abort = abort;
-    a.c11 = c[0].p;
-    a.c13 = c[1].p;
-    a.c33 = c[2].p;
+    a.c11 = c11;
+    a.c13 = c13;
+    a.c33 = c33;
     a.t0 = t0;
     a.tr = tr;
     return a;
 }
-
-}  // namespace
 
 int ResRun::setup(const std::vector<ShotB> &base, int nnz, int snap_fmt, const int *rxz, const int *r0, hipStream_t st)
 {
     std::vector<int> nnx;
     for (const ShotB &b : base) nnx.push_back(b.nnx);
     const int ns = (int)base.size();
-    int rc = setup_tiles(f, res_rows(nnx.data(), ns, nnz, false, snap_fmt), base, nnz, rxz, r0, st);
+    int rc = res_setup(f, res_rows(nnx.data(), ns, nnz, false, snap_fmt), base, nnz, rxz, r0, st);
     if (!rc && !lb.empty())
-        rc = setup_tiles(b, res_rows(nnx.data(), ns, nnz, true, snap_fmt), base, nnz, rxz, r0, st);
-    if (!rc) rc = upload(lfd, lf, st);
-    if (!rc) rc = upload(lbd, lb, st);
+        rc = res_setup(b, res_rows(nnx.data(), ns, nnz, true, snap_fmt), base, nnz, rxz, r0, st);
+    if (!rc) rc = res_upload(lfd, lf, st);
+    if (!rc) rc = res_upload(lbd, lb, st);
     if (!rc) rc = abortd.alloc(1, st);
     return rc;
 }
@@ -235,11 +148,10 @@ int ResRun::forward(const BatchGeo &bg, float dx2, float dz2, float dt2, const D
                     float *tr, int nt, bool taper_first, const SnapW &sw, int last_snap, hipStream_t st)
 {
     VTI_CHECK(active() && (int)lf.size() >= nt, "resident forward: not set up");
-    const ResArgs a = res_args(f, abortd.p, bg, dx2, dz2, dt2, c, t0, tr);
+    const ResArgs a = res_args(f, abortd.p, bg, dx2, dz2, dt2, c[0].p, c[1].p, c[2].p, t0, tr);
     const dim3 grid((unsigned)f.ntiles), block(64, kResNW);
     const int tf = taper_first ? 1 : 0;
-    return gated(st, [&] {
-        clear_halo(f.halo, st);
+    return res_launch(f.halo, st, [&] {
         with_rows(f.nr, [&](auto n) {
             if (sw.s16) fwd2d_res_kernel<n.value, 3><<<grid, block, 0, st>>>(a, lfd.p, nt, tf, sw, last_snap);
             else fwd2d_res_kernel<n.value, 0><<<grid, block, 0, st>>>(a, lfd.p, nt, tf, sw, last_snap);
@@ -252,11 +164,10 @@ int ResRun::adjoint(const BatchGeo &bg, float dx2, float dz2, float dt2, const D
                     hipStream_t st)
 {
     VTI_CHECK(active() && b.nr && (snap_fmt == 0 || snap_fmt == 3), "resident adjoint: not set up");
-    const ResArgs a = res_args(b, abortd.p, bg, dx2, dz2, dt2, c, t0, tr);
+    const ResArgs a = res_args(b, abortd.p, bg, dx2, dz2, dt2, c[0].p, c[1].p, c[2].p, t0, tr);
     const dim3 grid((unsigned)b.ntiles), block(64, kResNW);
     const int nlev = (int)lb.size();
-    return gated(st, [&] {
-        clear_halo(b.halo, st);
+    return res_launch(b.halo, st, [&] {
         with_rows(b.nr, [&](auto n) {
             if (snap_fmt == 3)
                 bwd2d_res_kernel<n.value, 3><<<grid, block, 0, st>>>(a, lbd.p, nlev, sr, last_row, g11, g13, g33);
@@ -266,15 +177,19 @@ int ResRun::adjoint(const BatchGeo &bg, float dx2, float dz2, float dt2, const D
     });
 }
 
-int ResRun::aborted(bool *yes, hipStream_t st) const
+int res_gave_up(const DBuf<int> &abort, bool *yes, hipStream_t st)
 {
-    *yes = false;
-    if (!active()) return kOk;
     int h = 0;
-    VTI_HIP(hipMemcpyAsync(&h, abortd.p, sizeof h, hipMemcpyDeviceToHost, st));
+    VTI_HIP(hipMemcpyAsync(&h, abort.p, sizeof h, hipMemcpyDeviceToHost, st));
     VTI_HIP(hipStreamSynchronize(st));
     *yes = h != 0;
     return kOk;
+}
+
+int ResRun::aborted(bool *yes, hipStream_t st) const
+{
+    *yes = false;
+    return active() ? res_gave_up(abortd, yes, st) : kOk;
 }
 
 }  // namespace vti

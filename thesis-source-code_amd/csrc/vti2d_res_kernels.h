@@ -25,7 +25,7 @@
 // level ahead cannot overwrite a word that is still to be read.
 //
 // All workgroups of a launch must be on the chip at once, since they wait for
-// one another: the host launches no more than fit (res_capacity) and one
+// one another: the host launches no more than fit (res_per_cu) and one
 // resident launch per device at a time.  Every wait is bounded: after
 // kResWait without its word (something else holds the CUs) a wavefront raises
 // the abort flag and waits no more, the others see the flag and do the same,
@@ -72,7 +72,8 @@ struct LevF {
     int pad;
 };
 
-// A receiver within its tile: point (row * 64 + column) and trace column.
+// A receiver within its tile: point (row * 64 + column) and trace column; ~ir
+// at the negative pole of a dipole receiver (the point below it).
 struct ResRec {
     int pt, ir;
 };
@@ -123,7 +124,8 @@ struct ResTile {
     unsigned wx, wu, wd;
     int lx;            // LDS place of the halo column value
 
-    __device__ __forceinline__ void init(const ResArgs &a, const ShotB &sh, int tile, int z0)
+    // nf: field pairs exchanged, each with strips of its own
+    __device__ __forceinline__ void init(const ResArgs &a, const ShotB &sh, int tile, int z0, int nf = 1)
     {
         const int tl = tile - sh.tile0, tx = tl % sh.ntx;
         lane = threadIdx.x;
@@ -133,7 +135,7 @@ struct ResTile {
         const int nact = min(D::TH, rows), below = rows - D::TH;
         nk = max(0, min(NR, nact - row0));
         const bool lf = tx > 0, rt = tx + 1 < sh.ntx, up = tl >= sh.ntx, dn = below > 0;
-        const unsigned own = 2u * D::WORDS * tile;
+        const unsigned tw = 2u * D::WORDS * nf, own = tw * tile;
         // lanes in the order of the strips' words: 4 NR of the left columns, 4 NR of the right ones
         const bool right = lane >= 4 * NR;
         const int r = row0 + ((right ? lane - 4 * NR : lane) >> 2), c = lane & 3;
@@ -145,12 +147,12 @@ struct ResTile {
         wt = own + D::T + row0 * 64 + lane;
         wb = own + D::B + (row0 - (D::TH - 4)) * 64 + lane;
         get_x = send_c;
-        wx = (right ? 2u * D::WORDS * (tile + 1) + D::L : 2u * D::WORDS * (tile - 1) + D::R) + 4 * r + c;
+        wx = (right ? tw * (tile + 1) + D::L : tw * (tile - 1) + D::R) + 4 * r + c;
         lx = r * D::PW + (right ? 68 : 0) + c;
         get_u = up;
-        wu = 2u * D::WORDS * (tile - sh.ntx) + D::B + w * 64 + lane;
+        wu = tw * (tile - sh.ntx) + D::B + w * 64 + lane;
         get_d = w < min(4, below);
-        wd = 2u * D::WORDS * (tile + sh.ntx) + D::T + w * 64 + lane;
+        wd = tw * (tile + sh.ntx) + D::T + w * 64 + lane;
     }
 };
 
@@ -359,7 +361,11 @@ struct ResTaper {
 // the source (objFuncGradient_f.cu:160-210, synthetic_f.cu:86-110), with the
 // source, the taper, the recorded traces and the D snapshots.
 // lev[it]: what level it does; last_snap: the slot of D of the last level.
-// SF: the snapshots' format (0 also for none).
+// SF: the snapshots' format (0 also for none); kResSlice: no D snapshots, but
+// 0.5 (p + q) of the recorded levels into the planes of sw.d
+// (recordWavefieldSlice, kernels.cu:335-343), one shot, from a dipole source.
+enum { kResSlice = 4 };
+
 template <int NR, int SF, int KIND>
 __device__ __forceinline__ void fwd2d_res_body(const ResArgs &A, const ResTile<NR> &t, const ShotB &sh,
                                                const ResTaper<NR> &tap, int tile, int x, int z0, float *lds,
@@ -376,7 +382,7 @@ __device__ __forceinline__ void fwd2d_res_body(const ResArgs &A, const ResTile<N
     // the two levels are those of the LDS planes; registers hold the coefficients
     float p[NR], q[NR], a11[NR], a13[NR], a33[NR];
     const float v1 = lev[1].src;
-    unsigned smask = 0;  // this lane's rows that hold the source
+    unsigned smask = 0, nmask = 0;  // this lane's rows that hold the source, a dipole's second pole
 #pragma unroll
     for (int k = 0; k < NR; ++k) {
         p[k] = q[k] = a11[k] = a13[k] = a33[k] = 0.f;
@@ -390,9 +396,14 @@ __device__ __forceinline__ void fwd2d_res_body(const ResArgs &A, const ResTile<N
                 p[k] = taper_first ? v1 * tap.template at<KIND>(k) : v1;
                 q[k] = p[k];
             }
+            if (SF == kResSlice && (int)(i0 + k * nnx) == sh.src + nnx) {
+                nmask |= 1u << k;
+                p[k] = -v1 * tap.template at<KIND>(k);
+                q[k] = p[k];
+            }
         }
     }
-    const bool has_src = __ballot(smask != 0) != 0;
+    const bool has_src = __ballot((smask | nmask) != 0) != 0;
     const int rec0 = A.rec_at[tile], rec1 = A.rec_at[tile + 1];
     auto record = [&](int it, int row) {
         const float *pr = pl(it) + 4, *qr = ql(it) + 4 * D::QW;
@@ -413,11 +424,20 @@ __device__ __forceinline__ void fwd2d_res_body(const ResArgs &A, const ResTile<N
             }
     };
     bool gone = false;
+    auto put_slice = [&](int slot) {
+        float *out = sw.d + (long long)slot * nnx * A.bg.nnz;
+#pragma unroll
+        for (int k = 0; k < NR; ++k)
+            if (k < nk && act) st32(out, i0 + k * nnx, 0.5f * (p[k] + q[k]));
+    };
     res_send<NR>(t, A.halo, pl(1), ql(1), p, q, 1);
     LevF l = lev[min(2, nt - 1)];
     res_recv<NR>(t, A.halo, A.abort, gone, pl(1), ql(1), 1);
     lds_barrier();
-    if (lev[1].row >= 0) record(1, lev[1].row);
+    if (lev[1].row >= 0) {
+        if (SF == kResSlice) put_slice(lev[1].row);
+        else record(1, lev[1].row);
+    }
     // Level it from the current (pc, qc) over the previous (p, q).  The next
     // level's entry is read ahead of the wait: a scalar load still in flight
     // holds up every LDS read after it.
@@ -436,6 +456,10 @@ __device__ __forceinline__ void fwd2d_res_body(const ResArgs &A, const ResTile<N
                 pn += cur.src;
                 qn += cur.src;
             }
+            if (SF == kResSlice && has_src && (nmask >> k & 1)) {
+                pn -= cur.src;
+                qn -= cur.src;
+            }
             const bool on = KIND != kResAny || (act && k < nk);
             p[k] = KIND == kResInner ? pn : on ? pn * tk : 0.f;
             q[k] = KIND == kResInner ? qn : on ? qn * tk : 0.f;
@@ -443,10 +467,14 @@ __device__ __forceinline__ void fwd2d_res_body(const ResArgs &A, const ResTile<N
         res_send<NR>(t, A.halo, pl(it), ql(it), p, q, it);
         __builtin_amdgcn_s_setprio(0);
         l = lev[min(it + 1, nt - 1)];
-        if (cur.snap >= 0) put_snap(cur.snap, tp, tq);
+        if (SF == kResSlice) {
+            if (cur.row >= 0) put_slice(cur.row);
+        } else if (cur.snap >= 0) {
+            put_snap(cur.snap, tp, tq);
+        }
         res_recv<NR>(t, A.halo, A.abort, gone, pl(it), ql(it), it);
         lds_barrier();
-        if (cur.row >= 0 && rec0 < rec1) record(it, cur.row);
+        if (SF != kResSlice && cur.row >= 0 && rec0 < rec1) record(it, cur.row);
     };
     for (int it = 2; it < nt; ++it) step(it);
     if (last_snap >= 0) {
@@ -691,6 +719,337 @@ static __global__ __launch_bounds__(64 * kResNW) __attribute__((amdgpu_waves_per
     else
         bwd2d_res_body<NR, SF, kResAny>(A, t, sh, tap, tile, x0 + t.lane, z0, lds, lev, nlev, sr, last_row, G11,
                                         G13, G33);
+}
+
+
+// Forward pass of GNhessian_f (hessian_f.cu:735-806): the background field as
+// above, and the Born field with the scattering source dt2 * (dC * D p)
+// (kernels.cu:282-291), which is the one recorded; the background's D snapshots
+// in FP32.  One shot.
+template <int NR, int KIND>
+__device__ __forceinline__ void born2d_res_body(const ResArgs &A, const ResTile<NR> &t, const ShotB &sh,
+                                                const ResTaper<NR> &tap, int tile, int x, int z0, float *lds,
+                                                const float *__restrict__ dc11, const float *__restrict__ dc13,
+                                                const float *__restrict__ dc33, const LevF *__restrict__ lev, int nt,
+                                                const SnapW &sw, int last_snap)
+{
+    using D = ResDim<NR>;
+    const int nnx = sh.nnx, tid = t.lane + 64 * t.w;
+    const int nk = KIND == kResAny ? t.nk : NR;
+    const bool act = KIND == kResAny ? x < nnx - 4 : true;
+    const unsigned i0 = x + (z0 + t.row0) * nnx;
+    constexpr int F = 2 * D::P + 2 * D::Q;  // the Born field's planes follow the background's
+    auto pl = [&](int it) { return lds + (it & 1) * D::P; };
+    auto ql = [&](int it) { return lds + 2 * D::P + (it & 1) * D::Q; };
+    ResTile<NR> tb = t;  // and so do its strips
+    tb.wc += 2 * D::WORDS;
+    tb.wt += 2 * D::WORDS;
+    tb.wb += 2 * D::WORDS;
+    tb.wx += 2 * D::WORDS;
+    tb.wu += 2 * D::WORDS;
+    tb.wd += 2 * D::WORDS;
+    float p[NR], q[NR], dp[NR], dq[NR], a11[NR], a13[NR], a33[NR], b11[NR], b13[NR], b33[NR];
+    unsigned smask = 0;
+#pragma unroll
+    for (int k = 0; k < NR; ++k) {
+        p[k] = q[k] = dp[k] = dq[k] = a11[k] = a13[k] = a33[k] = b11[k] = b13[k] = b33[k] = 0.f;
+        if (k < nk && act) {
+            const unsigned i = i0 + k * nnx;
+            a11[k] = A.c11[i];
+            a13[k] = A.c13[i];
+            a33[k] = A.c33[i];
+            b11[k] = dc11[i];
+            b13[k] = dc13[i];
+            b33[k] = dc33[i];
+            if ((int)i == sh.src) {
+                smask |= 1u << k;
+                p[k] = q[k] = lev[1].src;
+            }
+        }
+    }
+    const bool has_src = __ballot(smask != 0) != 0;
+    const int rec0 = A.rec_at[tile], rec1 = A.rec_at[tile + 1];
+    auto put_snap = [&](int slot, const float (&tp)[NR], const float (&tq)[NR]) {
+#pragma unroll
+        for (int k = 0; k < NR; ++k)
+            if (k < nk && act) snap_put32(sw, sh, (long long)nnx * A.bg.nnz, slot, i0 + k * nnx, tp[k], tq[k]);
+    };
+    bool gone = false;
+    res_send<NR>(t, A.halo, pl(1), ql(1), p, q, 1);
+    res_send<NR>(tb, A.halo, pl(1) + F, ql(1) + F, dp, dq, 1);
+    LevF l = lev[min(2, nt - 1)];
+    res_recv<NR>(t, A.halo, A.abort, gone, pl(1), ql(1), 1);
+    res_recv<NR>(tb, A.halo, A.abort, gone, pl(1) + F, ql(1) + F, 1);
+    lds_barrier();
+    for (int it = 2; it < nt; ++it) {
+        const LevF cur = l;
+        float tp[NR], tq[NR], bp[NR], bq[NR], pc[NR], qc[NR];
+        const int own_p = t.row0 * D::PW + t.lane + 4, own_q = (t.row0 + 4) * D::QW + t.lane;
+        res_d<NR>(t, A, pl(it - 1), ql(it - 1), nk, act, tp, tq, pc, qc);
+#pragma unroll
+        for (int k = 0; k < NR; ++k) {
+            const float tk = tap.template at<KIND>(k), pp = pl(it)[own_p + k * D::PW], qp = ql(it)[own_q + k * D::QW];
+            float pn = 2.f * pc[k] + A.dt2 * (a11[k] * tp[k] + a13[k] * tq[k]) - (KIND == kResInner ? pp : pp * tk);
+            float qn = 2.f * qc[k] + A.dt2 * (a13[k] * tp[k] + a33[k] * tq[k]) - (KIND == kResInner ? qp : qp * tk);
+            if (has_src && (smask >> k & 1)) {
+                pn += cur.src;
+                qn += cur.src;
+            }
+            const bool on = KIND != kResAny || (act && k < nk);
+            p[k] = KIND == kResInner ? pn : on ? pn * tk : 0.f;
+            q[k] = KIND == kResInner ? qn : on ? qn * tk : 0.f;
+        }
+        res_send<NR>(t, A.halo, pl(it), ql(it), p, q, it);
+        res_d<NR>(t, A, pl(it - 1) + F, ql(it - 1) + F, nk, act, bp, bq, pc, qc);
+#pragma unroll
+        for (int k = 0; k < NR; ++k) {
+            const float tk = tap.template at<KIND>(k), pp = (pl(it) + F)[own_p + k * D::PW],
+                        qp = (ql(it) + F)[own_q + k * D::QW];
+            float pn = 2.f * pc[k] + A.dt2 * (a11[k] * bp[k] + a13[k] * bq[k]) - (KIND == kResInner ? pp : pp * tk);
+            float qn = 2.f * qc[k] + A.dt2 * (a13[k] * bp[k] + a33[k] * bq[k]) - (KIND == kResInner ? qp : qp * tk);
+            pn += A.dt2 * (b11[k] * tp[k] + b13[k] * tq[k]);
+            qn += A.dt2 * (b13[k] * tp[k] + b33[k] * tq[k]);
+            const bool on = KIND != kResAny || (act && k < nk);
+            dp[k] = KIND == kResInner ? pn : on ? pn * tk : 0.f;
+            dq[k] = KIND == kResInner ? qn : on ? qn * tk : 0.f;
+        }
+        res_send<NR>(tb, A.halo, pl(it) + F, ql(it) + F, dp, dq, it);
+        l = lev[min(it + 1, nt - 1)];
+        if (cur.snap >= 0) put_snap(cur.snap, tp, tq);
+        res_recv<NR>(t, A.halo, A.abort, gone, pl(it), ql(it), it);
+        res_recv<NR>(tb, A.halo, A.abort, gone, pl(it) + F, ql(it) + F, it);
+        lds_barrier();
+        if (cur.row >= 0 && rec0 < rec1) {
+            const float *pr = pl(it) + F + 4, *qr = ql(it) + F + 4 * D::QW;
+            float *out = A.tr + sh.r_off + (long long)cur.row * sh.nr;
+            for (int e = rec0 + tid; e < rec1; e += 64 * kResNW) {
+                const ResRec r = A.rec[e];
+                out[r.ir] = 0.5f * (pr[(r.pt >> 6) * D::PW + (r.pt & 63)] + qr[r.pt]);
+            }
+        }
+    }
+    float tp[NR], tq[NR], pc[NR], qc[NR];
+    res_d<NR>(t, A, pl(nt - 1), ql(nt - 1), nk, act, tp, tq, pc, qc);
+    put_snap(last_snap, tp, tq);
+}
+
+template <int NR>
+static __global__ __launch_bounds__(64 * kResNW) __attribute__((amdgpu_waves_per_eu(NR == 6 ? 2 : 3))) void born2d_res_kernel(
+    ResArgs A, const float *__restrict__ dc11, const float *__restrict__ dc13, const float *__restrict__ dc33,
+    const LevF *__restrict__ lev, int nt, SnapW sw, int last_snap)
+{
+    using D = ResDim<NR>;
+    __shared__ float lds[4 * D::P + 4 * D::Q];
+    const int tid = threadIdx.x + 64 * threadIdx.y;
+    for (int k = tid; k < 4 * D::P + 4 * D::Q; k += 64 * kResNW) lds[k] = 0.f;
+    const int tile = xcd_tile();
+    const ShotB sh = A.shots[A.tile_shot[tile]];
+    const int tl = tile - sh.tile0;
+    const int x0 = 4 + (tl % sh.ntx) * 64, z0 = 4 + (tl / sh.ntx) * D::TH;
+    ResTile<NR> t;
+    t.init(A, sh, tile, z0, 2);
+    ResTaper<NR> tap;
+    const bool one = tap.init(A, sh, t, x0, z0), full = t.nk == NR && x0 + 64 <= sh.nnx - 4;
+    __syncthreads();
+    if (full && one)
+        born2d_res_body<NR, kResInner>(A, t, sh, tap, tile, x0 + t.lane, z0, lds, dc11, dc13, dc33, lev, nt, sw,
+                                       last_snap);
+    else if (full)
+        born2d_res_body<NR, kResFull>(A, t, sh, tap, tile, x0 + t.lane, z0, lds, dc11, dc13, dc33, lev, nt, sw,
+                                      last_snap);
+    else
+        born2d_res_body<NR, kResAny>(A, t, sh, tap, tile, x0 + t.lane, z0, lds, dc11, dc13, dc33, lev, nt, sw,
+                                     last_snap);
+}
+
+// Backward pass on the forward operator (forwardCD), one shot.  IMG 0:
+// GNhessian_f's adjoint (hessian_f.cu:834-900), the Born traces injected and
+// imaged as in the adjoint above.  IMG 1: rtm_f's receiver side
+// (rtm_f.cu:152-216), data injected as dipoles and
+// image += 0.5 (p + q) * the interpolated slice.
+// lev[n]: as for the adjoint; row < 0: nothing injected at this level.
+template <int NR, int IMG, int KIND>
+__device__ __forceinline__ void back2d_res_body(const ResArgs &A, const ResTile<NR> &t, const ShotB &sh,
+                                                const ResTaper<NR> &tap, int tile, int x, int z0, float *lds,
+                                                const LevelB *__restrict__ lev, int nlev,
+                                                const float *__restrict__ snap, int last_row, float *__restrict__ G11,
+                                                float *__restrict__ G13, float *__restrict__ G33)
+{
+    using D = ResDim<NR>;
+    constexpr int NI = IMG ? 1 : 3, NS = IMG ? 1 : 2;  // images, planes of a slot
+    const int nnx = sh.nnx;
+    const int nk = KIND == kResAny ? t.nk : NR;
+    const bool act = KIND == kResAny ? x < nnx - 4 : true;
+    const unsigned i0 = x + (z0 + t.row0) * nnx;
+    const long long plane = (long long)nnx * A.bg.nnz;
+    auto pl = [&](unsigned n) { return lds + (n & 1) * D::P; };
+    auto ql = [&](unsigned n) { return lds + 2 * D::P + (n & 1) * D::Q; };
+    float p[NR], q[NR], a11[NR], a13[NR], a33[NR], g[NI][NR], d0[NS][NR], d1[NS][NR];
+    unsigned rmask = 0, nmask = 0;  // rows with a receiver; those of a negative pole
+    int rbase = A.rec_at[tile];
+    const int rec1 = A.rec_at[tile + 1];
+    auto key = [&](int pt) { return (((pt >> 6) / NR) * 64 + (pt & 63)) * NR + (pt >> 6) % NR; };
+    for (int hi = rec1; rbase < hi;) {
+        const int m = (rbase + hi) >> 1;
+        if (key(A.rec[m].pt) < (t.w * 64 + t.lane) * NR) rbase = m + 1;
+        else hi = m;
+    }
+    auto column = [](int ir) { return ir < 0 ? ~ir : ir; };
+    int at = rbase;
+#pragma unroll
+    for (int k = 0; k < NR; ++k) {
+        p[k] = q[k] = a11[k] = a13[k] = a33[k] = 0.f;
+#pragma unroll
+        for (int j = 0; j < NI; ++j) g[j][k] = 0.f;
+#pragma unroll
+        for (int j = 0; j < NS; ++j) d0[j][k] = d1[j][k] = 0.f;
+        if (k < nk && act) {
+            a11[k] = A.c11[i0 + k * nnx];
+            a13[k] = A.c13[i0 + k * nnx];
+            a33[k] = A.c33[i0 + k * nnx];
+            if (at < rec1 && A.rec[at].pt == (t.row0 + k) * 64 + t.lane) {
+                const int ir = A.rec[at++].ir;
+                rmask |= 1u << k;
+                if (ir < 0) nmask |= 1u << k;
+                // the last row into zero fields; the taper follows in rtm_f alone
+                const float r0 = A.tr[(long long)last_row * sh.nr + column(ir)];
+                const float s = 0.5f * ((1.f - 0.f) * r0 + 0.f * 0.f), v = A.dt2 * s;
+                if (IMG) p[k] = ir < 0 ? -v * tap.template at<KIND>(k) : v * tap.template at<KIND>(k);
+                else p[k] += v;
+                q[k] = p[k];
+            }
+        }
+    }
+    const bool anyrec = __ballot(rmask != 0) != 0;
+    const int ir0 = rmask ? column(A.rec[rbase].ir) : 0;
+    int slot = -2;
+    auto load_slot = [&](int s, float (&d)[NS][NR]) {
+#pragma unroll
+        for (int j = 0; j < NS; ++j)
+#pragma unroll
+            for (int k = 0; k < NR; ++k)
+                if (k < nk && act) d[j][k] = ld32(snap + ((long long)s * NS + j) * plane, i0 + k * nnx);
+    };
+    auto slots = [&](int s) {
+        if (s == slot) return;
+        if (s == slot - 1) {
+#pragma unroll
+            for (int j = 0; j < NS; ++j)
+#pragma unroll
+                for (int k = 0; k < NR; ++k) d1[j][k] = d0[j][k];
+        } else {
+            load_slot(s + 1, d1);
+        }
+        load_slot(s, d0);
+        slot = s;
+    };
+    auto image = [&](float f) {
+#pragma unroll
+        for (int k = 0; k < NR; ++k) {
+            const float Dp = (1.f - f) * d0[0][k] + f * d1[0][k];
+            if (IMG) {
+                g[0][k] = g[0][k] + 0.5f * (p[k] + q[k]) * Dp;
+            } else {
+                const float Dq = (1.f - f) * d0[NS - 1][k] + f * d1[NS - 1][k];
+                g[0][k] = g[0][k] + p[k] * Dp;
+                g[NI / 2][k] = g[NI / 2][k] + (p[k] * Dq + q[k] * Dp);
+                g[NI - 1][k] = g[NI - 1][k] + q[k] * Dq;
+            }
+        }
+    };
+    bool gone = false;
+    res_send<NR>(t, A.halo, pl(1), ql(1), p, q, 1);
+    slots(lev[0].slot);
+    image(lev[0].f);
+    LevelB l = lev[min(1, nlev - 1)];
+    res_recv<NR>(t, A.halo, A.abort, gone, pl(1), ql(1), 1);
+    lds_barrier();
+    for (int n = 1; n < nlev; ++n) {
+        const LevelB cur = l;
+        const unsigned tag = n + 1;
+        slots(cur.slot);
+        const bool inject = anyrec && cur.row >= 0;
+        const float *row = A.tr + (long long)cur.row * sh.nr;
+        float r0 = 0.f, r1 = 0.f;
+        if (inject && rmask) {
+            r0 = row[ir0];
+            r1 = row[ir0 + sh.nr];
+        }
+        float tp[NR], tq[NR], pc[NR], qc[NR];
+        res_d<NR>(t, A, pl(n), ql(n), nk, act, tp, tq, pc, qc);
+        const float *pv = pl(tag) + t.row0 * D::PW + t.lane + 4, *qv = ql(tag) + (t.row0 + 4) * D::QW + t.lane;
+        int e = rbase;
+#pragma unroll
+        for (int k = 0; k < NR; ++k) {
+            const float tk = tap.template at<KIND>(k), pp = pv[k * D::PW], qp = qv[k * D::QW];
+            float pn = 2.f * pc[k] + A.dt2 * (a11[k] * tp[k] + a13[k] * tq[k]) - (KIND == kResInner ? pp : pp * tk);
+            float qn = 2.f * qc[k] + A.dt2 * (a13[k] * tp[k] + a33[k] * tq[k]) - (KIND == kResInner ? qp : qp * tk);
+            if (inject && (rmask >> k & 1)) {
+                if (e != rbase) {  // further receivers of the lane
+                    const int ir = column(A.rec[e].ir);
+                    r0 = row[ir];
+                    r1 = row[ir + sh.nr];
+                }
+                ++e;
+                const float s = 0.5f * ((1.f - cur.fr) * r0 + cur.fr * r1);
+                if (IMG && (nmask >> k & 1)) {
+                    pn -= A.dt2 * s;
+                    qn -= A.dt2 * s;
+                } else {
+                    pn += A.dt2 * s;
+                    qn += A.dt2 * s;
+                }
+            }
+            const bool on = KIND != kResAny || (act && k < nk);
+            p[k] = KIND == kResInner ? pn : on ? pn * tk : 0.f;
+            q[k] = KIND == kResInner ? qn : on ? qn * tk : 0.f;
+        }
+        if (n + 1 < nlev) res_send<NR>(t, A.halo, pl(tag), ql(tag), p, q, tag);
+        l = lev[min(n + 1, nlev - 1)];
+        image(cur.f);
+        if (n + 1 < nlev) {
+            res_recv<NR>(t, A.halo, A.abort, gone, pl(tag), ql(tag), tag);
+            lds_barrier();
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < NR; ++k)
+        if (k < nk && act) {
+            G11[i0 + k * nnx] = g[0][k];
+            if (!IMG) {
+                G13[i0 + k * nnx] = g[NI / 2][k];
+                G33[i0 + k * nnx] = g[NI - 1][k];
+            }
+        }
+}
+
+template <int NR, int IMG>
+static __global__ __launch_bounds__(64 * kResNW) __attribute__((amdgpu_waves_per_eu(3))) void back2d_res_kernel(
+    ResArgs A, const LevelB *__restrict__ lev, int nlev, const float *__restrict__ snap, int last_row,
+    float *__restrict__ G11, float *__restrict__ G13, float *__restrict__ G33)
+{
+    using D = ResDim<NR>;
+    __shared__ float lds[2 * D::P + 2 * D::Q];
+    const int tid = threadIdx.x + 64 * threadIdx.y;
+    for (int k = tid; k < 2 * D::P + 2 * D::Q; k += 64 * kResNW) lds[k] = 0.f;
+    const int tile = xcd_tile();
+    const ShotB sh = A.shots[A.tile_shot[tile]];
+    const int tl = tile - sh.tile0;
+    const int x0 = 4 + (tl % sh.ntx) * 64, z0 = 4 + (tl / sh.ntx) * D::TH;
+    ResTile<NR> t;
+    t.init(A, sh, tile, z0);
+    ResTaper<NR> tap;
+    const bool one = tap.init(A, sh, t, x0, z0), full = t.nk == NR && x0 + 64 <= sh.nnx - 4;
+    __syncthreads();
+    if (full && one)
+        back2d_res_body<NR, IMG, kResInner>(A, t, sh, tap, tile, x0 + t.lane, z0, lds, lev, nlev, snap, last_row, G11,
+                                            G13, G33);
+    else if (full)
+        back2d_res_body<NR, IMG, kResFull>(A, t, sh, tap, tile, x0 + t.lane, z0, lds, lev, nlev, snap, last_row, G11,
+                                           G13, G33);
+    else
+        back2d_res_body<NR, IMG, kResAny>(A, t, sh, tap, tile, x0 + t.lane, z0, lds, lev, nlev, snap, last_row, G11,
+                                          G13, G33);
 }
 
 }  // namespace vti

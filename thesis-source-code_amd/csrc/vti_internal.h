@@ -82,6 +82,34 @@ int grad2d_merged(vti_ctx *ctx, const Grad2dPart *p, int n, const float *wavelet
 // device: its forward pass, and with grad its adjoint
 bool res2d_fits(vti_ctx *ctx, int nnx, int nnz, bool grad);
 
+// One shot on a grid with the init_abc taper, its model and traces on the
+// device (vti2d_res1.hip): c11/c13/c33 at pitch nnx, tr time-major (nr a row),
+// rxz the receivers' (ix, iz).
+struct Res2dShot {
+    vti_ctx *ctx;
+    int nnx, nnz, npad, nt, ratio, nr;
+    long long src;
+    const int *rxz;
+    float dx2, dz2, dt2;
+    const float *c[3];
+    float *tr;
+};
+// Whether the passes fit the chip, and the passes: GNhessian_f's forward pass
+// (background and Born field, FP32 snapshots, the Born traces into tr) and its
+// adjoint (the gradient stored at interior points); the source side of rtm_f /
+// odcig_f (a dipole source, slices of 0.5 (p + q); scaled: every source value
+// carries dt^2); rtm_f's receiver side (the data of tr injected as dipoles,
+// the image stored at interior points; level it < nt_neg injects nothing).
+// *gone: a wait ran out, the results are void and the call is for the
+// per-level kernels.
+bool res2d_fits_gn(const Res2dShot &s);
+bool res2d_fits_slices(const Res2dShot &s);
+bool res2d_fits_image(const Res2dShot &s);
+int res2d_gn(const Res2dShot &s, const float *const *dc, const float *wavelet, float *snap, float *g11, float *g13,
+             float *g33, bool *gone);
+int res2d_slices(const Res2dShot &s, const float *wavelet, bool scaled, float *slices, bool *gone);
+int res2d_image(const Res2dShot &s, int nt_neg, int last_row, const float *slices, float *image, bool *gone);
+
 int dmalloc(void **p, size_t bytes, hipStream_t s);
 // free device memory of the current device, counting the large blocks
 // dmalloc keeps for reuse
