@@ -136,3 +136,23 @@ def test_rtm_vs_oracle(vti, orc, ctx):
     print(f"rtm rel vs FP64 oracle {rel(img, r64):.2e}", flush=True)
     assert np.array_equal(img, ref)
     assert rel(img, r64) < 1e-3
+
+
+@pytest.mark.parametrize("nz,ny,nx,npad", [(41, 36, 44, 1), (29, 33, 71, 14), (34, 30, 300, 9)])
+def test_shells_vs_oracle(vti, orc, ctx, nz, ny, nx, npad):
+    """The coefficient volumes get their shells on the device: packed values
+    that differ from the model's everywhere, from a shell one point thick to
+    one that leaves a single interior plane.  Equal to the oracle bit for bit."""
+    P = problem(nz=nz, ny=ny, nx=nx, npad=npad, nt=67, ns=1)
+    padb, randb = _boundaries(vti, P)
+    padb = (padb * np.random.default_rng(nx).uniform(0.8, 1.0, padb.size)).astype(np.float32)
+    obs = np.zeros(len(P["recloc"]) * ((P["nt"] - 1) // 4 + 1), np.float32)
+    args = (P["souloc"], np.arange(1), P["recloc"], P["w"])
+    rest = (P["nt"], npad, P["o"], P["d"], P["dt"], P["rate"], obs)
+    print("3d shells", nz, ny, nx, npad, flush=True)
+    cg, co = P["cij"].copy(), P["cij"].copy()
+    f, g = vti.objfunc_gradient3d(ctx, *args, cg, padb, randb, *rest)
+    fo, go = orc.gradient3d(orc.REF, *args, co, padb, randb, *rest)
+    assert np.abs(go).max() > 0
+    assert np.array_equal(g, go) and np.array_equal(cg, co)
+    assert abs(f - fo) <= 2e-7 * abs(fo)

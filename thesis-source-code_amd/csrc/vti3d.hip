@@ -9,11 +9,16 @@
 // profile, the traces and the accumulators.  This replaces the reference's
 // host-streamed, temporally blocked z-block pipeline
 // (objFuncGradient3d_f.cu:538-1078) while reproducing its results.
+#include <sys/mman.h>
+#include <unistd.h>
+
 #include <algorithm>
 #include <cmath>
+#include <cstdint>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <initializer_list>
 #include <vector>
 
 #include "vti3d_kernels.h"
@@ -159,10 +164,41 @@ __global__ void accumulate64_kernel(double *__restrict__ acc, const float *__res
         acc[i] += (double)v[i];
 }
 
-__global__ void narrow64_kernel(float *__restrict__ out, const double *__restrict__ acc, long long n)
+// The pitched accumulator rounded to float, in the reference's contiguous
+// layout.  Blocks take rows (y, z) in turn.
+__global__ void narrow64_kernel(float *__restrict__ out, const double *__restrict__ acc, Geo3 g)
 {
-    for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
-        out[i] = (float)acc[i];
+    for (long long r = blockIdx.x; r < (long long)g.ny * g.nz; r += gridDim.x) {
+        const double *a = acc + r * g.pitch;
+        for (int x = threadIdx.x; x < g.nx; x += blockDim.x) out[r * g.nx + x] = (float)a[x];
+    }
+}
+
+// putBoundary (boundary.cpp:48-84) on the way to the device layout: the
+// contiguous volume c with its shell of npad points taken from `packed`, whose
+// order is the top slab, for each interior plane the npad front rows, npad +
+// npad values of every interior row and the npad back rows, and the bottom
+// slab.  Blocks take rows (y, z) in turn.
+__global__ void shell3d_kernel(float *__restrict__ dst, const float *__restrict__ c,
+                               const float *__restrict__ packed, Geo3 g, int npad)
+{
+    const int mx = g.nx - 2 * npad, my = g.ny - 2 * npad, mz = g.nz - 2 * npad;
+    const long long nxy = (long long)g.nx * g.ny, per = nxy - (long long)mx * my;  // per: of an interior plane
+    for (long long r = blockIdx.x; r < (long long)g.ny * g.nz; r += gridDim.x) {
+        const int z = (int)(r / g.ny), y = (int)(r % g.ny);
+        const int zi = z - npad, yi = y - npad;
+        const bool slab = zi < 0 || zi >= mz, whole = slab || yi < 0 || yi >= my;
+        long long at = zi < 0 ? z * nxy : npad * nxy + min(zi, mz) * per + max(zi - mz, 0) * nxy;
+        if (slab || yi < 0) at += (long long)y * g.nx;
+        else at += (long long)npad * g.nx + 2LL * npad * min(yi, my) + (long long)max(yi - my, 0) * g.nx;
+        for (int x = threadIdx.x; x < g.nx; x += blockDim.x) {
+            float v;
+            if (whole || x < npad) v = packed[at + x];
+            else if (x >= npad + mx) v = packed[at + x - mx];
+            else v = c[r * g.nx + x];
+            dst[r * g.pitch + x] = v;
+        }
+    }
 }
 
 }  // namespace
@@ -188,6 +224,7 @@ struct vti3d_prop {
     int zc = 64;
     int arith = 1;  // kArithRef
     size_t bytes = 0;
+    std::vector<void *> blocks;  // what the volumes were allocated as
     // two forward levels per launch: the second buffer pair it writes, and
     // whether their values outside the updated interior match (sx[1], sz[1])
     // and (sx[0], sz[0]) -- any other write to the fields clears it
@@ -244,52 +281,66 @@ int prop_free(vti3d_prop *p)
     (void)hipSetDevice(p->ctx->device);
     (void)hipStreamSynchronize(p->ctx->stream);
     hipStream_t s = p->ctx->stream;
-    for (int k = 0; k < 3; ++k) {
-        freep(p->cm[0][k], s);
-        freep(p->cm[1][k], s);
-        freep(p->acc[k], s);
-        freep(p->acc64[k], s);
-    }
-    freep(p->dxy, s);
-    freep(p->dzv, s);
-    for (int k = 0; k < 2; ++k) {
-        freep(p->sx[k], s);
-        freep(p->sz[k], s);
-        freep(p->lx[k], s);
-        freep(p->lz[k], s);
-        freep(p->sx2[k], s);
-        freep(p->sz2[k], s);
-    }
+    for (void *q : p->blocks) freep(q, s);
     (void)hipStreamSynchronize(s);
     delete p;
     return vti::kOk;
 }
 
-template <class T>
-int dalloc(vti3d_prop *p, T **ptr, size_t n)
+// One array a propagator holds: where its address goes and its size, a
+// multiple of 256 bytes for all but the last of a list.
+struct Part {
+    void **at;
+    size_t bytes;
+};
+
+// The arrays of `parts` that are not there yet, zeroed.  Small volumes are cut
+// from one block: an allocation and its release cost 0.1 to 0.15 ms each below
+// the size from which the library keeps blocks for reuse, 3.5 ms of a 17.8 ms
+// migration of 163 x 140 x 128 points.  Volumes of that size stay blocks of
+// their own, which fit whatever is released and asked for next.
+constexpr size_t kOwnBlock = size_t(64) << 20;
+int dalloc(vti3d_prop *p, std::initializer_list<Part> parts)
 {
-    if (*ptr) return vti::kOk;
-    const int rc = vti::dmalloc((void **)ptr, n * sizeof(T), p->ctx->stream);
-    if (rc) return rc;
-    p->bytes += n * sizeof(T);
-    VTI_HIP(hipMemsetAsync(*ptr, 0, n * sizeof(T), p->ctx->stream));
+    const hipStream_t s = p->ctx->stream;
+    size_t shared = 0;
+    for (const Part &a : parts)
+        if (!*a.at && a.bytes < kOwnBlock) shared += a.bytes;
+    char *base = nullptr;
+    if (shared) {
+        const int rc = vti::dmalloc((void **)&base, shared, s);
+        if (rc) return rc;
+        p->blocks.push_back(base);
+        p->bytes += shared;
+        VTI_HIP(hipMemsetAsync(base, 0, shared, s));
+    }
+    for (const Part &a : parts) {
+        if (*a.at) continue;
+        if (a.bytes < kOwnBlock) {
+            *a.at = base;
+            base += a.bytes;
+            continue;
+        }
+        const int rc = vti::dmalloc(a.at, a.bytes, s);
+        if (rc) return rc;
+        p->blocks.push_back(*a.at);
+        p->bytes += a.bytes;
+        VTI_HIP(hipMemsetAsync(*a.at, 0, a.bytes, s));
+    }
     return vti::kOk;
 }
 
 // lambda fields and accumulators are only needed by the backward passes
 int ensure_backward(vti3d_prop *p, bool gradient, bool random_model)
 {
-    const size_t nv = (size_t)vox(p->g);
-    int rc = vti::kOk;
-    for (int k = 0; k < 2 && rc == vti::kOk; ++k) {
-        rc = dalloc(p, &p->lx[k], nv);
-        if (rc == vti::kOk) rc = dalloc(p, &p->lz[k], nv);
-    }
-    for (int k = 0; k < (gradient ? 3 : 1) && rc == vti::kOk; ++k) {
-        rc = dalloc(p, &p->acc[k], nv);
-        if (rc == vti::kOk) rc = dalloc(p, &p->acc64[k], nv);
-    }
-    for (int k = 0; k < 3 && random_model && rc == vti::kOk; ++k) rc = dalloc(p, &p->cm[1][k], nv);
+    const size_t f = (size_t)vox(p->g) * sizeof(float), d = 2 * f;
+    auto at = [](auto **q) { return (void **)q; };
+    int rc = dalloc(p, {{at(&p->lx[0]), f}, {at(&p->lz[0]), f}, {at(&p->lx[1]), f}, {at(&p->lz[1]), f},
+                        {at(&p->acc[0]), f}, {at(&p->acc64[0]), d}});
+    if (rc == vti::kOk && gradient)
+        rc = dalloc(p, {{at(&p->acc[1]), f}, {at(&p->acc64[1]), d}, {at(&p->acc[2]), f}, {at(&p->acc64[2]), d}});
+    if (rc == vti::kOk && random_model)
+        rc = dalloc(p, {{at(&p->cm[1][0]), f}, {at(&p->cm[1][1]), f}, {at(&p->cm[1][2]), f}});
     return rc;
 }
 
@@ -421,11 +472,10 @@ void fwd_t2_kernel(vti3d_prop *p, const Launch &L, long long src_dev, float v1, 
 int fwd2_launch(vti3d_prop *p, bool absorbing, long long src_dev, float v1, float v2)
 {
     const size_t nv = (size_t)vox(p->g);
-    for (int k = 0; k < 2; ++k) {
-        int rc = dalloc(p, &p->sx2[k], nv);
-        if (!rc) rc = dalloc(p, &p->sz2[k], nv);
-        if (rc) return rc;
-    }
+    const size_t f = nv * sizeof(float);
+    const int rc = dalloc(p, {{(void **)&p->sx2[0], f}, {(void **)&p->sz2[0], f}, {(void **)&p->sx2[1], f},
+                              {(void **)&p->sz2[1], f}});
+    if (rc) return rc;
     if (!p->t2_synced) {
         VTI_HIP(hipMemcpyAsync(p->sx2[0], p->sx[1], nv * 4, hipMemcpyDeviceToDevice, p->ctx->stream));
         VTI_HIP(hipMemcpyAsync(p->sz2[0], p->sz[1], nv * 4, hipMemcpyDeviceToDevice, p->ctx->stream));
@@ -652,6 +702,7 @@ int backward_pass(vti3d_prop *p, int mode, int lmax, int nt, const float *wavele
     return vti::kOk;
 }
 
+int row_blocks(const Geo3 &g) { return (int)std::min<long long>(1 << 16, (long long)g.ny * g.nz); }
 int launch_blocks(long long n) { return (int)std::min<long long>(4096, std::max<long long>(1, (n + 255) / 256)); }
 
 }  // namespace
@@ -698,15 +749,11 @@ int vti3d_prop_create(vti_ctx *ctx, vti3d_prop **out, int nx, int ny, int nz, in
         delete p;
         VTI_CHECK(false, "vti3d_prop_create: x-y plane %dx%d too large for 32-bit chunk offsets", nx, ny);
     }
-    const size_t nv = (size_t)vox(g);
-    int rc = vti::kOk;
-    for (int k = 0; k < 3 && rc == vti::kOk; ++k) rc = dalloc(p, &p->cm[0][k], nv);
-    for (int k = 0; k < 2 && rc == vti::kOk; ++k) {
-        rc = dalloc(p, &p->sx[k], nv);
-        if (rc == vti::kOk) rc = dalloc(p, &p->sz[k], nv);
-    }
-    if (rc == vti::kOk) rc = dalloc(p, &p->dxy, (size_t)g.plane);
-    if (rc == vti::kOk) rc = dalloc(p, &p->dzv, (size_t)nz);
+    const size_t f = (size_t)vox(g) * sizeof(float);
+    int rc = dalloc(p, {{(void **)&p->cm[0][0], f}, {(void **)&p->cm[0][1], f}, {(void **)&p->cm[0][2], f},
+                        {(void **)&p->sx[0], f}, {(void **)&p->sz[0], f}, {(void **)&p->sx[1], f},
+                        {(void **)&p->sz[1], f}, {(void **)&p->dxy, (size_t)g.plane * sizeof(float)},
+                        {(void **)&p->dzv, (size_t)nz * sizeof(float)}});
     if (rc != vti::kOk) {
         prop_free(p);
         return rc;
@@ -1094,19 +1141,43 @@ int modeled_shot(vti3d_prop *p, const DriverArgs &a, const Shot3 &sh, ShotDev &s
     return vti::kOk;
 }
 
-int put_shell_and_upload(vti3d_prop *p, float *const dst[3], const float *cij, const float *packed, int nx, int ny,
-                         int nz, int npad)
+// The three coefficient volumes with their shells put on the device: set 0
+// takes `pad`'s, set 1, if asked for, `rand`'s.  The host arrays go over as
+// they are, into wavefield volumes that the first shot clears: putting the
+// shells on a host copy of each volume and uploading the six of them took 59
+// ms of a 152 ms gradient call at 239 x 283 x 232 points; with this and
+// map_pages the call takes 94.
+int upload_shelled(vti3d_prop *p, const float *cij, const float *pad, const float *rand)
 {
-    const long long nxyz = (long long)nx * ny * nz, nb = vti::boundary_size(nx, ny, nz, npad);
-    std::vector<float> tmp((size_t)nxyz);
+    const Geo3 &g = p->g;
+    const long long nxyz = (long long)g.nx * g.ny * g.nz, nb = vti::boundary_size(g.nx, g.ny, g.nz, p->npad);
+    hipStream_t s = p->ctx->stream;
+    const float *packed[2] = {pad, rand};
     for (int k = 0; k < 3; ++k) {
-        std::memcpy(tmp.data(), cij + k * nxyz, sizeof(float) * nxyz);
-        if (packed) vti::put_boundary(packed + k * nb, tmp.data(), nx, ny, nz, npad);
-        int rc = upload_volume(p, dst[k], tmp.data());
-        if (rc) return rc;
-        VTI_HIP(hipStreamSynchronize(p->ctx->stream));
+        VTI_HIP(hipMemcpyAsync(p->sx[0], cij + k * nxyz, sizeof(float) * nxyz, hipMemcpyHostToDevice, s));
+        for (int m = 0; m < (rand ? 2 : 1); ++m) {
+            VTI_HIP(hipMemcpyAsync(p->sz[0], packed[m] + k * nb, sizeof(float) * nb, hipMemcpyHostToDevice, s));
+            hipLaunchKernelGGL(shell3d_kernel, dim3(row_blocks(g)), dim3(256), 0, s, p->cm[m][k], p->sx[0], p->sz[0], g,
+                               p->npad);
+            VTI_HIP(hipGetLastError());
+        }
     }
+    VTI_HIP(hipStreamSynchronize(s));
     return vti::kOk;
+}
+
+// Has the kernel map the pages of a result that is to be written whole, while
+// the device still works on it.  Their contents stay; where this cannot be
+// done the copy maps them as it goes (18 ms for 188 MB of fresh memory).
+void map_pages(float *q, size_t n)
+{
+#ifdef MADV_POPULATE_WRITE
+    const uintptr_t page = (uintptr_t)sysconf(_SC_PAGESIZE);
+    const uintptr_t a = ((uintptr_t)q + page - 1) / page * page, b = (uintptr_t)(q + n) / page * page;
+    if (b > a) (void)madvise((void *)a, b - a, MADV_POPULATE_WRITE);
+#else
+    (void)q, (void)n;
+#endif
 }
 
 int accumulate(vti3d_prop *p, int n)
@@ -1121,13 +1192,21 @@ int accumulate(vti3d_prop *p, int n)
     return vti::kOk;
 }
 
-int narrow_download(vti3d_prop *p, float *dst, int k)
+// The first n accumulators to the caller's contiguous volumes, by way of the
+// wavefield volumes, which the last shot is done with; returns when they are there.
+int narrow_download(vti3d_prop *p, float *dst, int n)
 {
-    const long long nv = vox(p->g);
-    hipLaunchKernelGGL(narrow64_kernel, dim3(launch_blocks(nv)), dim3(256), 0, p->ctx->stream, p->acc[k], p->acc64[k],
-                       nv);
-    VTI_HIP(hipGetLastError());
-    return download_volume(p, dst, p->acc[k]);
+    const Geo3 &g = p->g;
+    const long long nxyz = (long long)g.nx * g.ny * g.nz;
+    float *stage[3] = {p->sx[0], p->sz[0], p->sx[1]};
+    for (int k = 0; k < n; ++k) {
+        hipLaunchKernelGGL(narrow64_kernel, dim3(row_blocks(g)), dim3(256), 0, p->ctx->stream, stage[k], p->acc64[k], g);
+        VTI_HIP(hipGetLastError());
+    }
+    for (int k = 0; k < n; ++k)
+        VTI_HIP(hipMemcpyAsync(dst + k * nxyz, stage[k], sizeof(float) * nxyz, hipMemcpyDeviceToHost, p->ctx->stream));
+    VTI_HIP(hipStreamSynchronize(p->ctx->stream));
+    return vti::kOk;
 }
 
 struct PropGuard {
@@ -1218,10 +1297,8 @@ static int objfunc_impl(vti_ctx *ctx, float *fgcij, bool grad, const float *soul
     if (grad) {
         rc = ensure_backward(p, true, true);
         if (rc) return rc;
-        rc = put_shell_and_upload(p, p->cm[1], cij, randboundaryCij, nx, ny, nz, npad);
-        if (rc) return rc;
     }
-    rc = put_shell_and_upload(p, p->cm[0], cij, padboundaryCij, nx, ny, nz, npad);
+    rc = upload_shelled(p, cij, padboundaryCij, grad ? randboundaryCij : nullptr);
     if (rc) return rc;
     const int sts = (int)std::round(samplingRate / dt), nnt = (nt - 1) / sts + 1, lmax = levels(nt, ngpu);
     VTI_CHECK(objtype == 0 || (halfwidth >= 0 && 2 * halfwidth < nnt),
@@ -1260,20 +1337,16 @@ static int objfunc_impl(vti_ctx *ctx, float *fgcij, bool grad, const float *soul
     }
     const long long nxyz = (long long)nx * ny * nz;
     fgcij[0] = (float)(objfunc / 2);
-    if (grad) {
-        for (int k = 0; k < 3; ++k) {
-            rc = narrow_download(p, fgcij + 1 + k * nxyz, k);
-            if (rc) return rc;
-        }
-        VTI_HIP(hipStreamSynchronize(p->ctx->stream));
-    }
-    // leave the caller's cij as the reference does (putBoundary in place)
+    // leave the caller's cij as the reference does (putBoundary in place); the
+    // device is still at the last backward pass, and what follows needs no
+    // more memory
+    if (grad) map_pages(fgcij + 1, 3 * nxyz);
     if (nshot > 0) {
         const long long nb = vti::boundary_size(nx, ny, nz, npad);
         const float *shell = grad ? randboundaryCij : padboundaryCij;
         for (int k = 0; k < 3; ++k) vti::put_boundary(shell + k * nb, cij + k * nxyz, nx, ny, nz, npad);
     }
-    return vti::kOk;
+    return grad ? narrow_download(p, fgcij + 1, 3) : vti::kOk;
 }
 
 int vti3d_objfunc_gradient(vti_ctx *ctx, float *fgcij, const float *souloc, int ns, const int *shotid, int nshot,
@@ -1367,12 +1440,10 @@ int vti3d_rtm(vti_ctx *ctx, float *image, const float *souloc, int ns, const int
         if (rc) return rc;
         rc = accumulate(p, 1);
         if (rc) return rc;
-        VTI_HIP(hipStreamSynchronize(p->ctx->stream));
+        if (k + 1 < nshot) VTI_HIP(hipStreamSynchronize(p->ctx->stream));
     }
-    rc = narrow_download(p, image, 0);
-    if (rc) return rc;
-    VTI_HIP(hipStreamSynchronize(p->ctx->stream));
-    return vti::kOk;
+    map_pages(image, (size_t)nx * ny * nz);
+    return narrow_download(p, image, 1);
 }
 
 }  // extern "C"

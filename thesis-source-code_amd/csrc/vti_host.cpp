@@ -26,9 +26,11 @@ void init_damping3d(float *damping, int nx, int ny, int nz, int npad)
         else dist = 0.f;
         return (float)(kDamper3D + (1. - kDamper3D) * std::cos(kPi3D * (double)dist / npad));
     };
+    std::vector<float> along_x(nx);
+    for (int ix = 0; ix < nx; ix++) along_x[ix] = profile(ix, nx);
     for (int iy = 0; iy < ny; iy++) {
         const float dy = profile(iy, ny);
-        for (int ix = 0; ix < nx; ix++) damping[ix + (size_t)iy * nx] = profile(ix, nx) * dy;
+        for (int ix = 0; ix < nx; ix++) damping[ix + (size_t)iy * nx] = along_x[ix] * dy;
     }
     const size_t nxy = (size_t)nx * ny;
     for (int iz = 0; iz < nz; iz++) damping[nxy + iz] = profile(iz, nz);
