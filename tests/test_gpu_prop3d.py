@@ -105,3 +105,52 @@ def test_two_levels_equal_one_level(vti, ctx, arith, absorbing):
             else:
                 for a, b in zip(out, ref):
                     assert np.array_equal(a, b), (nsteps, levels, zc)
+
+
+def _damping(vti, shape, npad):
+    """d = dxy * dz of every point the steps update, 1 elsewhere (the
+    propagator holds prev / d of the absorbing side)."""
+    nz, ny, nx = shape
+    d = vti.init_damping3d(nx, ny, nz, npad)
+    out = np.ones(shape, np.float32)
+    inner = np.s_[: 4 * (nz // 4), 4:ny - 4, 4:nx - 4]
+    out[inner] = (d[: nx * ny].reshape(ny, nx)[None] * d[nx * ny:][:, None, None]).astype(np.float32)[inner]
+    return out
+
+
+@pytest.mark.parametrize("arith", [1, 0], ids=["ref-arith", "fp32-arith"])
+@pytest.mark.parametrize("kind,dims", [("fwd", (430, 401, 15)), ("grad", (297, 290, 15)), ("rtm", (300, 345, 13))])
+def test_streamed_steps_vs_oracle(vti, orc, ctx, kind, dims, arith):
+    """Volumes whose rows fill a fifth of their pitch, so that a step's volumes
+    pass the size from which it streams past the caches: 4 levels, bit for bit."""
+    c, npad, n = _problem(*dims, seed=5), 5, 4
+    rng = np.random.default_rng(dims[1])
+    sig, lam = ([(rng.standard_normal(dims) * s).astype(np.float32) for _ in range(4)] for s in (1e-3, 1e-6))
+    dd = _damping(vti, dims, npad)
+    geo = (npad, 12.5, 12.5, 12.5, 1e-3)
+    print("streamed", kind, dims, arith, flush=True)
+    mode = 1 if kind == "rtm" else 0
+    with vti.Prop3D(ctx, dims[2], dims[1], dims[0], *geo) as p:
+        p.set_arith(arith)
+        p.set_model(*c)
+        p.set_state(cur_x=sig[0], cur_z=sig[2], prev_x=sig[1], prev_z=sig[3])
+        if kind == "fwd":
+            p.forward_steps(n, absorbing=True)
+        else:
+            p.set_adjoint(mode, cur_x=lam[0], cur_z=lam[2], prev_x=lam[1], prev_z=lam[3])
+            p.backward_steps(n, mode=mode)
+            la = p.get_adjoint(mode)
+        st = p.get_state()
+    if kind == "fwd":
+        o = [sig[0], sig[1] * dd, sig[2], sig[3] * dd]
+        orc.steps3d(orc.REF if arith else orc.F32, o, *c, *geo, n, absorbing=True)
+        st = [st[0], st[1], st[2] * dd, st[3] * dd]
+    else:
+        acc = [np.zeros(dims, np.float32) for _ in range(3 if mode == 0 else 1)]
+        o, lo = orc.bwd_steps3d(mode, arith, sig, [lam[0], lam[1] * dd, lam[2], lam[3] * dd], acc, *c, *geo, n)
+        for a, b in zip([la[0], la[1], la[2] * dd, la[3] * dd], (lo[0], lo[2], lo[1], lo[3])):
+            assert np.abs(b).max() > 0 and np.array_equal(a, b)
+        for a, b in zip(la[4], acc):
+            assert np.abs(b).max() > 0 and np.array_equal(a, b)
+    for a, b in zip(st, (o[0], o[2], o[1], o[3])):
+        assert np.abs(b).max() > 0 and np.array_equal(a, b)

@@ -19,6 +19,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <initializer_list>
+#include <type_traits>
 #include <vector>
 
 #include "vti3d_kernels.h"
@@ -421,25 +422,43 @@ Launch launch_shape(const vti3d_prop *p)
     return L;
 }
 
-template <int ARITH, bool ABC>
+// Whether a step that touches this many float volumes streams what it reads or
+// writes once a point past the caches.  Above the 288 MB that the Infinity
+// Cache and the L2s hold together it does (239 x 283 x 232: forward 108 us
+// against 127, gradient 281 against 314); below, the next level finds most of
+// it there (163 x 140 x 128: forward 25.7 us against 27.4, gradient 50 against
+// 59, RTM 47 against 53).  The two sides meet between 290 and 400 MB.
+bool streams(const vti3d_prop *p, int volumes)
+{
+    return 4 * volumes * vox(p->g) > (288LL << 20);
+}
+
+template <int ARITH, bool ABC, bool NT>
 void fwd_kernel(vti3d_prop *p, const Launch &L, long long src_dev, float src_val)
 {
-    hipLaunchKernelGGL((vti::fwd3d_kernel<ARITH, ABC, kBY>), L.grid, L.block, 0, p->ctx->stream, p->sx[1], p->sx[0],
-                       p->sz[1], p->sz[0], p->cm[p->active][0], p->cm[p->active][1], p->cm[p->active][2], p->dxy,
-                       p->dzv, p->g, p->zc, L.ntx, L.nty, p->dt2dx2, p->dt2dy2, p->dt2dz2, src_dev, src_val);
+    hipLaunchKernelGGL((vti::fwd3d_kernel<ARITH, ABC, kBY, NT>), L.grid, L.block, 0, p->ctx->stream, p->sx[1],
+                       p->sx[0], p->sz[1], p->sz[0], p->cm[p->active][0], p->cm[p->active][1], p->cm[p->active][2],
+                       p->dxy, p->dzv, p->g, p->zc, L.ntx, L.nty, p->dt2dx2, p->dt2dy2, p->dt2dz2, src_dev, src_val);
+}
+
+// f(std::true_type or std::false_type) for a run-time flag
+template <class F>
+void with_flag(bool b, F &&f)
+{
+    if (b) f(std::true_type{});
+    else f(std::false_type{});
 }
 
 int fwd_launch(vti3d_prop *p, bool absorbing, long long src_dev, float src_val)
 {
     p->t2_synced = false;
     const Launch L = launch_shape(p);
-    if (p->arith == vti::kArithRef) {
-        if (absorbing) fwd_kernel<vti::kArithRef, true>(p, L, src_dev, src_val);
-        else fwd_kernel<vti::kArithRef, false>(p, L, src_dev, src_val);
-    } else {
-        if (absorbing) fwd_kernel<vti::kArithF32, true>(p, L, src_dev, src_val);
-        else fwd_kernel<vti::kArithF32, false>(p, L, src_dev, src_val);
-    }
+    with_flag(absorbing, [&](auto abc) {
+        with_flag(streams(p, 7), [&](auto nt) {
+            if (p->arith == vti::kArithRef) fwd_kernel<vti::kArithRef, abc, nt>(p, L, src_dev, src_val);
+            else fwd_kernel<vti::kArithF32, abc, nt>(p, L, src_dev, src_val);
+        });
+    });
     VTI_HIP(hipGetLastError());
     std::swap(p->sx[0], p->sx[1]);
     std::swap(p->sz[0], p->sz[1]);
@@ -505,10 +524,10 @@ int fwd2_launch(vti3d_prop *p, bool absorbing, long long src_dev, float v1, floa
     return vti::kOk;
 }
 
-template <int MODE, int ARITH>
+template <int MODE, int ARITH, bool NT>
 void bwd_kernel(vti3d_prop *p, const Launch &L, long long src_dev, float src_val, int zrec0)
 {
-    hipLaunchKernelGGL((vti::bwd3d_kernel<MODE, ARITH, kBY>), L.grid, L.block, 0, p->ctx->stream, p->sx[1], p->sx[0],
+    hipLaunchKernelGGL((vti::bwd3d_kernel<MODE, ARITH, kBY, NT>), L.grid, L.block, 0, p->ctx->stream, p->sx[1], p->sx[0],
                        p->sz[1], p->sz[0], p->lx[1], p->lx[0], p->lz[1], p->lz[0], p->cm[p->active][0],
                        p->cm[p->active][1], p->cm[p->active][2], p->acc[0], MODE == 0 ? p->acc[1] : nullptr, MODE == 0 ? p->acc[2] : nullptr, p->dxy, p->dzv,
                        p->g, p->zc, L.ntx, L.nty, p->dx2, p->dy2, p->dz2, p->dt2, p->dt2dx2, p->dt2dy2, p->dt2dz2,
@@ -523,13 +542,13 @@ int bwd_launch(vti3d_prop *p, int mode, long long src_dev, float src_val, int zr
     p->t2_synced = false;
     const Geo3 &g = p->g;
     const Launch L = launch_shape(p);
-    if (p->arith == vti::kArithRef) {
-        if (mode == 0) bwd_kernel<0, vti::kArithRef>(p, L, src_dev, src_val, zrec0);
-        else bwd_kernel<1, vti::kArithRef>(p, L, src_dev, src_val, zrec0);
-    } else {
-        if (mode == 0) bwd_kernel<0, vti::kArithF32>(p, L, src_dev, src_val, zrec0);
-        else bwd_kernel<1, vti::kArithF32>(p, L, src_dev, src_val, zrec0);
-    }
+    with_flag(streams(p, mode == 0 ? 14 : 12), [&](auto nt) {
+        with_flag(mode == 0, [&](auto grad) {
+            constexpr int m = grad ? 0 : 1;
+            if (p->arith == vti::kArithRef) bwd_kernel<m, vti::kArithRef, nt>(p, L, src_dev, src_val, zrec0);
+            else bwd_kernel<m, vti::kArithF32, nt>(p, L, src_dev, src_val, zrec0);
+        });
+    });
     VTI_HIP(hipGetLastError());
     if (zrec0 >= 0) {
         if (nr > 0) {

@@ -71,6 +71,8 @@ __device__ __forceinline__ void bstore(rsrc_t r, unsigned lane_byte, unsigned un
 // streams a step touches once per point -- the previous level it overwrites,
 // the coefficients, the accumulators -- so that they do not displace the
 // sigma planes whose halo rows neighbouring workgroups read again from L2.
+// The step kernels take it as NT, off where the volumes of a step fit the
+// caches and the next level would find them there.
 constexpr int kNonTemporal = 2;
 __device__ __forceinline__ float bload_nt(rsrc_t r, unsigned lane_byte, unsigned uni_byte)
 {
@@ -79,6 +81,18 @@ __device__ __forceinline__ float bload_nt(rsrc_t r, unsigned lane_byte, unsigned
 __device__ __forceinline__ void bstore_nt(rsrc_t r, unsigned lane_byte, unsigned uni_byte, float v)
 {
     __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, (int)lane_byte, (int)uni_byte, kNonTemporal);
+}
+
+template <bool NT>
+__device__ __forceinline__ float bload_once(rsrc_t r, unsigned lane_byte, unsigned uni_byte)
+{
+    return NT ? bload_nt(r, lane_byte, uni_byte) : bload(r, lane_byte, uni_byte);
+}
+template <bool NT>
+__device__ __forceinline__ void bstore_once(rsrc_t r, unsigned lane_byte, unsigned uni_byte, float v)
+{
+    if (NT) bstore_nt(r, lane_byte, uni_byte, v);
+    else bstore(r, lane_byte, uni_byte, v);
 }
 
 template <int BY>
@@ -310,7 +324,7 @@ __device__ __forceinline__ void effective_column_rt(float *e, const float *q, fl
 // planes of requests outstanding.  Plane bases are wave-uniform; per-lane
 // offsets within a plane are 32-bit.
 // ---------------------------------------------------------------------------
-template <int ARITH, bool ABC, int BY>
+template <int ARITH, bool ABC, int BY, bool NT>
 __global__ __launch_bounds__(64 * BY) void fwd3d_kernel(
     float *__restrict__ nxt_x, const float *__restrict__ cur_x, float *__restrict__ nxt_z,
     const float *__restrict__ cur_z, const float *__restrict__ c11, const float *__restrict__ c13,
@@ -355,11 +369,11 @@ __global__ __launch_bounds__(64 * BY) void fwd3d_kernel(
     // point data of plane z (prev and coefficients)
     float px = 0.f, pz = 0.f, a11 = 0.f, a13 = 0.f, a33 = 0.f;
     if (inrange) {
-        px = bload_nt(Rnx, col4, so(zs));
-        pz = bload_nt(Rnz, col4, so(zs));
-        a11 = bload_nt(R11, col4, so(zs));
-        a13 = bload_nt(R13, col4, so(zs));
-        a33 = bload_nt(R33, col4, so(zs));
+        px = bload_once<NT>(Rnx, col4, so(zs));
+        pz = bload_once<NT>(Rnz, col4, so(zs));
+        a11 = bload_once<NT>(R11, col4, so(zs));
+        a13 = bload_once<NT>(R13, col4, so(zs));
+        a33 = bload_once<NT>(R33, col4, so(zs));
     }
     PlaneRegs<BY> P;
     P.loadb(Rcx, so(zs), L);
@@ -378,11 +392,11 @@ __global__ __launch_bounds__(64 * BY) void fwd3d_kernel(
             float npx = 0.f, npz = 0.f, n11 = 0.f, n13 = 0.f, n33 = 0.f, qn = 0.f;
             if (nx1) {
                 const unsigned o1 = so(z + 1);
-                npx = bload_nt(Rnx, col4, o1);
-                npz = bload_nt(Rnz, col4, o1);
-                n11 = bload_nt(R11, col4, o1);
-                n13 = bload_nt(R13, col4, o1);
-                n33 = bload_nt(R33, col4, o1);
+                npx = bload_once<NT>(Rnx, col4, o1);
+                npz = bload_once<NT>(Rnz, col4, o1);
+                n11 = bload_once<NT>(R11, col4, o1);
+                n13 = bload_once<NT>(R13, col4, o1);
+                n33 = bload_once<NT>(R33, col4, o1);
             }
             if (inrange && z + 5 < g.zmax) qn = bload(Rcz, col4, so(z + 5));
 
@@ -410,8 +424,8 @@ __global__ __launch_bounds__(64 * BY) void fwd3d_kernel(
                 vz = vz * d;
             }
             if (active) {
-                bstore_nt(Rnx, col4, so(z), vx);
-                bstore_nt(Rnz, col4, so(z), vz);
+                bstore_once<NT>(Rnx, col4, so(z), vx);
+                bstore_once<NT>(Rnz, col4, so(z), vz);
             }
             __syncthreads();
 #pragma unroll
@@ -782,7 +796,7 @@ __global__ __launch_bounds__(1024) void fwd3d_t2b_kernel(
 // the reference performs before damping is applied next by
 // inject_damp3d_kernel, which then damps those planes.
 // ---------------------------------------------------------------------------
-template <int MODE, int ARITH, int BY>
+template <int MODE, int ARITH, int BY, bool NT>
 __global__ __launch_bounds__(64 * BY) __attribute__((amdgpu_waves_per_eu(4))) void bwd3d_kernel(
     float *__restrict__ s_nx, const float *__restrict__ s_cx, float *__restrict__ s_nz,
     const float *__restrict__ s_cz, float *__restrict__ l_nx, const float *__restrict__ l_cx,
@@ -837,13 +851,13 @@ __global__ __launch_bounds__(64 * BY) __attribute__((amdgpu_waves_per_eu(4))) vo
     float spx = 0.f, spz = 0.f, lpx = 0.f, lpz = 0.f, a11 = 0.f, a13 = 0.f, a33 = 0.f;
     if (inrange) {
         const unsigned o0 = so(zs);
-        spx = bload_nt(Rsnx, col4, o0);
-        spz = bload_nt(Rsnz, col4, o0);
-        lpx = bload_nt(Rlnx, col4, o0);
-        lpz = bload_nt(Rlnz, col4, o0);
-        a11 = bload_nt(R11, col4, o0);
-        a13 = bload_nt(R13, col4, o0);
-        a33 = bload_nt(R33, col4, o0);
+        spx = bload_once<NT>(Rsnx, col4, o0);
+        spz = bload_once<NT>(Rsnz, col4, o0);
+        lpx = bload_once<NT>(Rlnx, col4, o0);
+        lpz = bload_once<NT>(Rlnz, col4, o0);
+        a11 = bload_once<NT>(R11, col4, o0);
+        a13 = bload_once<NT>(R13, col4, o0);
+        a33 = bload_once<NT>(R33, col4, o0);
     }
     PlaneRegs<BY> PS, PL;
     PS.loadb(Rscx, so(zs), L);
@@ -872,23 +886,23 @@ __global__ __launch_bounds__(64 * BY) __attribute__((amdgpu_waves_per_eu(4))) vo
             float o11 = 0.f, o13 = 0.f, o33 = 0.f;
             if (inrange) {
                 const unsigned oz = so(z);
-                o11 = bload_nt(G11, col4, oz);
+                o11 = bload_once<NT>(G11, col4, oz);
                 if (MODE == 0) {
-                    o13 = bload_nt(G13, col4, oz);
-                    o33 = bload_nt(G33, col4, oz);
+                    o13 = bload_once<NT>(G13, col4, oz);
+                    o33 = bload_once<NT>(G33, col4, oz);
                 }
             }
             float n_spx = 0.f, n_spz = 0.f, n_lpx = 0.f, n_lpz = 0.f, n11 = 0.f, n13 = 0.f, n33 = 0.f;
             float qsn = 0.f, qln = 0.f;
             if (inrange && z + 1 < ze) {
                 const unsigned o1 = so(z + 1);
-                n_spx = bload_nt(Rsnx, col4, o1);
-                n_spz = bload_nt(Rsnz, col4, o1);
-                n_lpx = bload_nt(Rlnx, col4, o1);
-                n_lpz = bload_nt(Rlnz, col4, o1);
-                n11 = bload_nt(R11, col4, o1);
-                n13 = bload_nt(R13, col4, o1);
-                n33 = bload_nt(R33, col4, o1);
+                n_spx = bload_once<NT>(Rsnx, col4, o1);
+                n_spz = bload_once<NT>(Rsnz, col4, o1);
+                n_lpx = bload_once<NT>(Rlnx, col4, o1);
+                n_lpz = bload_once<NT>(Rlnz, col4, o1);
+                n11 = bload_once<NT>(R11, col4, o1);
+                n13 = bload_once<NT>(R13, col4, o1);
+                n33 = bload_once<NT>(R33, col4, o1);
             }
             if (inrange && z + 5 < g.zmax) {
                 qsn = bload(Rscz, col4, so(z + 5));
@@ -944,14 +958,14 @@ __global__ __launch_bounds__(64 * BY) __attribute__((amdgpu_waves_per_eu(4))) vo
             }
             if (active) {
                 const unsigned oz = so(z);
-                bstore_nt(Rsnx, col4, oz, svx);
-                bstore_nt(Rsnz, col4, oz, svz);
-                bstore_nt(Rlnx, col4, oz, lvx);
-                bstore_nt(Rlnz, col4, oz, lvz);
-                bstore_nt(G11, col4, oz, o11);
+                bstore_once<NT>(Rsnx, col4, oz, svx);
+                bstore_once<NT>(Rsnz, col4, oz, svz);
+                bstore_once<NT>(Rlnx, col4, oz, lvx);
+                bstore_once<NT>(Rlnz, col4, oz, lvz);
+                bstore_once<NT>(G11, col4, oz, o11);
                 if (MODE == 0) {
-                    bstore_nt(G13, col4, oz, o13);
-                    bstore_nt(G33, col4, oz, o33);
+                    bstore_once<NT>(G13, col4, oz, o13);
+                    bstore_once<NT>(G33, col4, oz, o33);
                 }
             }
             __syncthreads();
