@@ -156,3 +156,27 @@ def test_shells_vs_oracle(vti, orc, ctx, nz, ny, nx, npad):
     assert np.abs(go).max() > 0
     assert np.array_equal(g, go) and np.array_equal(cg, co)
     assert abs(f - fo) <= 2e-7 * abs(fo)
+
+
+@pytest.mark.parametrize("edge", [False, True], ids=["interior", "outside"])
+def test_receiver_planes_vs_oracle(vti, orc, ctx, edge):
+    """Receivers in each of the four planes of their block, the first and the
+    last interior column among them ("outside": one past the updated interior,
+    which takes the injection as a launch of its own).  Bit for bit."""
+    P = problem(nz=40, ny=25, nx=71, npad=6, nt=131, ns=1)
+    d = P["d"][0]
+    for k in range(len(P["recloc"])):
+        P["recloc"][k, 2] = (8 + k % 4) * d + 0.1
+    if edge:
+        P["recloc"][2, 0] = d + 0.1
+    padb, randb = _boundaries(vti, P)
+    obs = _obs(vti, ctx, P)
+    print("3d receiver planes", edge, flush=True)
+    rest = (P["nt"], P["npad"], P["o"], P["d"], P["dt"], P["rate"])
+    args = (P["souloc"], np.arange(1), P["recloc"], P["w"])
+    _, g = vti.objfunc_gradient3d(ctx, *args, P["cij"].copy(), padb, randb, *rest, np.zeros_like(obs))
+    _, go = orc.gradient3d(orc.REF, *args, P["cij"].copy(), padb, randb, *rest, np.zeros_like(obs))
+    assert np.abs(go).max() > 0 and np.array_equal(g, go)
+    args = (P["souloc"], np.arange(1), np.ascontiguousarray(P["recloc"][:, :3]), P["w"], *P["cij"], *rest, obs)
+    img, ref = vti.rtm3d(ctx, *args), orc.rtm3d(orc.REF, *args)
+    assert np.abs(ref).max() > 0 and np.array_equal(img, ref)

@@ -423,14 +423,15 @@ Launch launch_shape(const vti3d_prop *p)
 }
 
 // Whether a step that touches this many float volumes streams what it reads or
-// writes once a point past the caches.  Above the 288 MB that the Infinity
+// writes once a point past the caches.  Well above the 288 MB that the Infinity
 // Cache and the L2s hold together it does (239 x 283 x 232: forward 108 us
 // against 127, gradient 281 against 314); below, the next level finds most of
 // it there (163 x 140 x 128: forward 25.7 us against 27.4, gradient 50 against
-// 59, RTM 47 against 53).  The two sides meet between 290 and 400 MB.
+// 59, RTM 47 against 53).  The two sides meet at 315 MB for the forward step
+// and near 400 for the other two (at 308 the gradient takes 86 us against 99).
 bool streams(const vti3d_prop *p, int volumes)
 {
-    return 4 * volumes * vox(p->g) > (288LL << 20);
+    return 4 * volumes * vox(p->g) > (320LL << 20);
 }
 
 template <int ARITH, bool ABC, bool NT>
@@ -525,19 +526,21 @@ int fwd2_launch(vti3d_prop *p, bool absorbing, long long src_dev, float v1, floa
 }
 
 template <int MODE, int ARITH, bool NT>
-void bwd_kernel(vti3d_prop *p, const Launch &L, long long src_dev, float src_val, int zrec0)
+void bwd_kernel(vti3d_prop *p, const Launch &L, long long src_dev, float src_val, int zrec0, const vti::Inject &rec)
 {
     hipLaunchKernelGGL((vti::bwd3d_kernel<MODE, ARITH, kBY, NT>), L.grid, L.block, 0, p->ctx->stream, p->sx[1], p->sx[0],
                        p->sz[1], p->sz[0], p->lx[1], p->lx[0], p->lz[1], p->lz[0], p->cm[p->active][0],
-                       p->cm[p->active][1], p->cm[p->active][2], p->acc[0], MODE == 0 ? p->acc[1] : nullptr, MODE == 0 ? p->acc[2] : nullptr, p->dxy, p->dzv,
+                       p->cm[p->active][1], p->cm[p->active][2], p->acc[0], MODE == 0 ? p->acc[1] : nullptr,
+                       MODE == 0 ? p->acc[2] : nullptr, p->dxy, p->dzv,
                        p->g, p->zc, L.ntx, L.nty, p->dx2, p->dy2, p->dz2, p->dt2, p->dt2dx2, p->dt2dy2, p->dt2dz2,
-                       src_dev, src_val, zrec0);
+                       src_dev, src_val, zrec0, rec);
 }
 
-// One backward level: the fused kernel, then (when the receiver block is
-// present) the injection and damping of the receiver planes.
-int bwd_launch(vti3d_prop *p, int mode, long long src_dev, float src_val, int zrec0, const long long *d_rec_eff,
-               const float *coarse, int nr, int i1, float f)
+// One backward level: the fused kernel and, where the nr receivers in `at`
+// have no map, the injection and damping of their planes.  zrec0 < 0: no
+// receiver planes.
+int bwd_launch(vti3d_prop *p, int mode, long long src_dev, float src_val, int zrec0, const vti::Inject &rec,
+               const long long *at, int nr)
 {
     p->t2_synced = false;
     const Geo3 &g = p->g;
@@ -545,17 +548,15 @@ int bwd_launch(vti3d_prop *p, int mode, long long src_dev, float src_val, int zr
     with_flag(streams(p, mode == 0 ? 14 : 12), [&](auto nt) {
         with_flag(mode == 0, [&](auto grad) {
             constexpr int m = grad ? 0 : 1;
-            if (p->arith == vti::kArithRef) bwd_kernel<m, vti::kArithRef, nt>(p, L, src_dev, src_val, zrec0);
-            else bwd_kernel<m, vti::kArithF32, nt>(p, L, src_dev, src_val, zrec0);
+            if (p->arith == vti::kArithRef) bwd_kernel<m, vti::kArithRef, nt>(p, L, src_dev, src_val, zrec0, rec);
+            else bwd_kernel<m, vti::kArithF32, nt>(p, L, src_dev, src_val, zrec0, rec);
         });
     });
     VTI_HIP(hipGetLastError());
-    if (zrec0 >= 0) {
-        if (nr > 0) {
-            hipLaunchKernelGGL(vti::inject_res3d_kernel, dim3((nr + 255) / 256), dim3(256), 0, p->ctx->stream,
-                               p->lx[1], p->lz[1], d_rec_eff, coarse, nr, i1, f, p->dt2);
-            VTI_HIP(hipGetLastError());
-        }
+    if (zrec0 >= 0 && !rec.map) {
+        hipLaunchKernelGGL(vti::inject_res3d_kernel, dim3((nr + 255) / 256), dim3(256), 0, p->ctx->stream, p->lx[1],
+                           p->lz[1], at, rec, nr, p->dt2);
+        VTI_HIP(hipGetLastError());
         hipLaunchKernelGGL(vti::damp_planes3d_kernel, dim3((g.nx + 255) / 256, g.ny, 4), dim3(256), 0,
                            p->ctx->stream, p->lx[1], p->lz[1], p->dxy, p->dzv, g, zrec0);
         VTI_HIP(hipGetLastError());
@@ -635,6 +636,7 @@ struct ShotDev {
     float *obs = nullptr;      // trace-major [nr][nnt]
     unsigned char *live = nullptr;
     double *partial = nullptr;
+    int *map = nullptr;  // the receivers in their planes (backward_pass)
     hipStream_t s;  // the stream that uses (and releases) them
     explicit ShotDev(hipStream_t st) : s(st) {}
     ~ShotDev()
@@ -646,6 +648,7 @@ struct ShotDev {
         freep(obs, s);
         freep(live, s);
         freep(partial, s);
+        freep(map, s);
     }
 };
 
@@ -692,30 +695,51 @@ int forward_pass(vti3d_prop *p, bool absorbing, int lmax, const float *wavelet, 
     return vti::kOk;
 }
 
+// True where no two receivers share a point and all lie in the updated
+// interior, so that each can be injected and damped at its own point.
+bool receivers_apart(const Geo3 &g, std::vector<long long> at)
+{
+    for (const long long i : at) {
+        const long long ix = i % g.nx, iy = i / g.nx % g.ny;
+        if (ix < 4 || ix >= g.nx - 4 || iy < 4 || iy >= g.ny - 4) return false;
+    }
+    std::sort(at.begin(), at.end());
+    return std::adjacent_find(at.begin(), at.end()) == at.end();
+}
+
 // Backward pass (gradient mode 0, RTM mode 1) after the random-boundary
 // forward and the flip: s = 2..lmax, it = nt-1-s, source dt2*wavelet[it+1],
 // receiver-side injection of the traces in sd.tr interpolated at it+1.
-int backward_pass(vti3d_prop *p, int mode, int lmax, int nt, const float *wavelet, long long sou_ref,
-                  const ShotDev &sd, int nr, int rec_block, int sts, int nnt)
+int backward_pass(vti3d_prop *p, int mode, int lmax, int nt, const float *wavelet, const Shot3 &sh, ShotDev &sd,
+                  int sts, int nnt)
 {
-    const long long src = dev_index(p->g, sou_ref);
-    const int zrec0 = 4 * rec_block;
-    const bool recv_ok = zrec0 + 3 < p->g.zmax;
+    const Geo3 &g = p->g;
+    const hipStream_t st = p->ctx->stream;
+    const long long src = dev_index(g, sh.sou_ref);
+    const int nr = sh.nr;
+    int zrec0 = 4 * sh.rec_block;
+    if (zrec0 + 3 >= g.zmax || nr == 0) zrec0 = -8;
+    if (zrec0 >= 0 && receivers_apart(g, sh.rec_eff)) {
+        const size_t bytes = sizeof(int) * 4 * (size_t)g.plane;
+        DMALLOC(&sd.map, bytes);
+        VTI_HIP(hipMemsetAsync(sd.map, 0, bytes, st));
+        hipLaunchKernelGGL(vti::receiver_map3d_kernel, dim3((nr + 255) / 256), dim3(256), 0, st, sd.map, sd.rec_eff,
+                           nr, zrec0 * g.plane);
+        VTI_HIP(hipGetLastError());
+    }
     for (int s = 2; s <= lmax; ++s) {
-        const int it = nt - 1 - s;
-        const int ti = it + 1;
-        float f = (float)ti / (float)sts;
-        int i1 = (int)f;
-        const float *coarse = sd.tr;
+        const int ti = nt - s;
+        const float f = (float)ti / (float)sts;
+        const int i1 = (int)f;
+        vti::Inject rec{sd.map, nullptr, nullptr, 0.f};
         if (i1 >= nnt - 1) {
-            coarse = sd.tr + (size_t)(nnt - 1) * nr;
-            i1 = -1;
-            f = 0.f;
+            rec.lo = sd.tr + (size_t)(nnt - 1) * nr;
         } else {
-            f = f - i1;
+            rec.lo = sd.tr + (size_t)i1 * nr;
+            rec.hi = rec.lo + nr;
+            rec.f = f - i1;
         }
-        int rc = bwd_launch(p, mode, src, p->dt2 * wavelet[it + 1], recv_ok ? zrec0 : -8, sd.rec_eff, coarse, nr, i1,
-                            f);
+        const int rc = bwd_launch(p, mode, src, p->dt2 * wavelet[ti], zrec0, rec, sd.rec_eff, nr);
         if (rc) return rc;
     }
     return vti::kOk;
@@ -1001,7 +1025,7 @@ int vti3d_prop_backward_steps(vti3d_prop *p, int mode, int nsteps, float *elapse
         VTI_HIP(hipEventRecord(e0, p->ctx->stream));
     }
     for (int s = 0; s < nsteps; ++s) {
-        rc = bwd_launch(p, mode, -1, 0.f, -8, nullptr, nullptr, 0, 0, 0.f);
+        rc = bwd_launch(p, mode, -1, 0.f, -8, vti::Inject{}, nullptr, 0);
         if (rc) return rc;
     }
     if (elapsed_ms) {
@@ -1349,7 +1373,7 @@ static int objfunc_impl(vti_ctx *ctx, float *fgcij, bool grad, const float *soul
             hipLaunchKernelGGL(lambda_init3d_kernel, dim3((sh.nr + 255) / 256), dim3(256), 0, p->ctx->stream,
                                p->lx[0], p->lz[0], sd.rec_true, sd.tr + (size_t)(nnt - 1) * sh.nr, sh.nr, p->dt2);
         VTI_HIP(hipGetLastError());
-        rc = backward_pass(p, 0, lmax, nt, wavelet, sh.sou_ref, sd, sh.nr, sh.rec_block, sts, nnt);
+        rc = backward_pass(p, 0, lmax, nt, wavelet, sh, sd, sts, nnt);
         if (rc) return rc;
         rc = accumulate(p, 3);
         if (rc) return rc;
@@ -1455,7 +1479,7 @@ int vti3d_rtm(vti_ctx *ctx, float *image, const float *souloc, int ns, const int
             hipLaunchKernelGGL(lambda_init3d_kernel, dim3((sh.nr + 255) / 256), dim3(256), 0, p->ctx->stream,
                                p->lx[0], p->lz[0], sd.rec_true, sd.tr + (size_t)(nnt - 1) * sh.nr, sh.nr, p->dt2);
         VTI_HIP(hipGetLastError());
-        rc = backward_pass(p, 1, lmax, nt, wavelet, sh.sou_ref, sd, sh.nr, sh.rec_block, sts, nnt);
+        rc = backward_pass(p, 1, lmax, nt, wavelet, sh, sd, sts, nnt);
         if (rc) return rc;
         rc = accumulate(p, 1);
         if (rc) return rc;

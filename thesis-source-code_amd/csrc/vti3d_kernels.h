@@ -780,6 +780,32 @@ __global__ __launch_bounds__(1024) void fwd3d_t2b_kernel(
     }
 }
 
+// Residual (or observed-data) injection into lambda_next at the receivers
+// (injectResidual, injectRecord3d.cu:38-46) with the time interpolation of
+// interpolateResidual (injectRecord3d.cu:60-78) evaluated on the device.
+struct Inject {
+    const int *map;         // receiver + 1 or 0 at each point of the four receiver planes; null: a launch of its own
+    const float *lo, *hi;   // the two coarse samples' rows, one value a receiver; hi null: lo as it is
+    float f;
+};
+
+__device__ __forceinline__ void inject(const Inject &in, int ir, float dt2, float &lx, float &lz)
+{
+    float fine = in.lo[ir];
+    if (in.hi) fine = (float)((1. - (double)in.f) * (double)fine + (double)(in.f * in.hi[ir]));
+    const float s = dt2 * fine;
+    lx = (float)((double)lx + VTI_TWOTHIRD_D * (double)s);
+    lz = (float)((double)lz + VTI_ONETHIRD_D * (double)s);
+}
+
+// map of a shot's receivers, no two at one point; first: the index of the first receiver plane
+__global__ void receiver_map3d_kernel(int *__restrict__ map, const long long *__restrict__ rec, int nr,
+                                      long long first)
+{
+    const int ir = blockIdx.x * blockDim.x + threadIdx.x;
+    if (ir < nr) map[rec[ir] - first] = ir + 1;
+}
+
 // ---------------------------------------------------------------------------
 // Fused backward step of the 3D gradient and RTM passes.
 //
@@ -791,10 +817,13 @@ __global__ __launch_bounds__(1024) void fwd3d_t2b_kernel(
 // MODE 1 (RTM, rtm3d_f.cu:585-610): forwardKernel on both fields and
 //   image += (2/3 sx + 1/3 sz)(2/3 lx + 1/3 lz), with lambda at the current
 //   level after its damping.
-// The source injection into sigma_next is fused (own point).  In the four
-// receiver planes lambda_next is stored undamped: the residual injection that
-// the reference performs before damping is applied next by
-// inject_damp3d_kernel, which then damps those planes.
+// The source injection into sigma_next is fused (own point), and so is the
+// receivers' into lambda_next, which the reference performs before the
+// damping: the four receiver planes are stored undamped, and at its end a
+// workgroup that marched through them takes its points there again, each with
+// its receiver from rec.map.  (Inside the march that costs 20 to 30 scalar
+// registers too many.)  Without a map it is left to two launches, which take
+// 10 us a level.
 // ---------------------------------------------------------------------------
 template <int MODE, int ARITH, int BY, bool NT>
 __global__ __launch_bounds__(64 * BY) __attribute__((amdgpu_waves_per_eu(4))) void bwd3d_kernel(
@@ -804,12 +833,14 @@ __global__ __launch_bounds__(64 * BY) __attribute__((amdgpu_waves_per_eu(4))) vo
     const float *__restrict__ c13, const float *__restrict__ c33, float *__restrict__ g11, float *__restrict__ g13,
     float *__restrict__ g33, const float *__restrict__ dxy_plane, const float *__restrict__ dzv, Geo3 g, int zc,
     int ntx, int nty, float dx2, float dy2, float dz2, float dt2, float dt2dx2, float dt2dy2, float dt2dz2,
-    long long src_idx, float src_val, int zrec0)
+    long long src_idx, float src_val, int zrec0, Inject rec_arg)
 {
     constexpr int W = Tile<BY>::W;
     constexpr int R = Tile<BY>::R;
     __shared__ float ts[2][R * W];
     __shared__ float tl[2][R * W];
+    __shared__ Inject rec;  // waits here for the end: the march is short of scalar registers
+    if (threadIdx.x == 0 && threadIdx.y == 0) rec = rec_arg;
 
     const int lb = xcd_logical_block(gridDim.x * gridDim.y * gridDim.z);
     const int bx = lb % ntx, by = (lb / ntx) % nty, bz = lb / (ntx * nty);
@@ -985,29 +1016,34 @@ __global__ __launch_bounds__(64 * BY) __attribute__((amdgpu_waves_per_eu(4))) vo
             a33 = n33;
         }
     }
+
+    // the receiver planes, all four in one chunk: each thread's own points again
+    if (active && zrec0 >= zs && zrec0 < ze && rec.map) {
+        const Inject in = rec;
+        for (int k = 0; k < 4; ++k) {
+            const unsigned oz = so(zrec0 + k);
+            const int ir = in.map[(size_t)k * (pb / 4) + L.main_off] - 1;
+            const float d = dxy * dzv[zrec0 + k];
+            float lvx = bload(Rlnx, col4, oz), lvz = bload(Rlnz, col4, oz);
+            if (ir >= 0) inject(in, ir, dt2, lvx, lvz);
+            bstore(Rlnx, col4, oz, lvx * d);
+            bstore(Rlnz, col4, oz, lvz * d);
+        }
+    }
 }
 
-// Residual (or observed-data) injection into lambda_next at the receivers
-// (injectResidual, injectRecord3d.cu:38-46) with the time interpolation of
-// interpolateResidual (injectRecord3d.cu:60-78) evaluated on the device:
-// the coarse traces are time-major rows [it][ir]; i1 < 0 selects row nnt-1.
+// The injection on its own, with the damping of the receiver planes after it,
+// where receivers share a point or lie outside the updated interior.
 __global__ void inject_res3d_kernel(float *__restrict__ lx, float *__restrict__ lz,
-                                    const long long *__restrict__ rec, const float *__restrict__ coarse, int nr,
-                                    int i1, float f, float dt2)
+                                    const long long *__restrict__ rec, Inject in, int nr, float dt2)
 {
     const int ir = blockIdx.x * blockDim.x + threadIdx.x;
     if (ir >= nr) return;
-    float fine;
-    if (i1 < 0) {
-        fine = coarse[ir];
-    } else {
-        fine = (float)((1. - (double)f) * (double)coarse[(size_t)i1 * nr + ir] +
-                       (double)(f * coarse[(size_t)(i1 + 1) * nr + ir]));
-    }
-    const float s = dt2 * fine;
     const long long i = rec[ir];
-    lx[i] = (float)((double)lx[i] + VTI_TWOTHIRD_D * (double)s);
-    lz[i] = (float)((double)lz[i] + VTI_ONETHIRD_D * (double)s);
+    float x = lx[i], z = lz[i];
+    inject(in, ir, dt2, x, z);
+    lx[i] = x;
+    lz[i] = z;
 }
 
 // Damping of the four receiver planes after the injection (abcXYZ/abcXY).
