@@ -154,3 +154,28 @@ def test_streamed_steps_vs_oracle(vti, orc, ctx, kind, dims, arith):
             assert np.abs(b).max() > 0 and np.array_equal(a, b)
     for a, b in zip(st, (o[0], o[2], o[1], o[3])):
         assert np.abs(b).max() > 0 and np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("dims", [(8, 9, 9), (16, 17, 71), (19, 75, 133), (36, 25, 390)])
+def test_tile_order_vs_oracle(vti, orc, ctx, dims):
+    """1 to 63 tiles a z-chunk, fewer than the XCDs and no multiple of them, in
+    1 to 9 chunks: every tile of every chunk is stepped once."""
+    c, npad, n = _problem(*dims, seed=dims[2]), 3, 3
+    rng = np.random.default_rng(dims[1])
+    st = [(rng.standard_normal(dims) * 1e-3).astype(np.float32) for _ in range(4)]
+    geo = (npad, 12.5, 12.5, 12.5, 1e-3)
+    print("tile order", dims, flush=True)
+    want = [a.copy() for a in st]
+    orc.steps3d(orc.REF, want, *c, *geo, n, absorbing=False)
+    for levels, zc in ((1, 0), (1, 8), (2, 4)):
+        with vti.Prop3D(ctx, dims[2], dims[1], dims[0], *geo) as p:
+            p.set_levels(levels)
+            if zc:
+                p.set_zchunk(zc)
+            p.set_model(*c)
+            p.set_state(cur_x=st[0], cur_z=st[2], prev_x=st[1], prev_z=st[3])
+            p.forward_steps(n, absorbing=False)
+            got = p.get_state()
+        # 3 levels (odd): the oracle's arrays have changed roles
+        for a, b in zip(got, (want[1], want[3], want[0], want[2])):
+            assert np.abs(b).max() > 0 and np.array_equal(a, b)

@@ -222,7 +222,7 @@ struct vti3d_prop {
     float *lx[2] = {nullptr, nullptr}, *lz[2] = {nullptr, nullptr};
     float *acc[3] = {nullptr, nullptr, nullptr};  // per-shot gradient (or image in acc[0])
     double *acc64[3] = {nullptr, nullptr, nullptr};
-    int zc = 64;
+    int zc = 0, zc2 = 0;  // z-chunk of the one-level and of the two-level launches
     int arith = 1;  // kArithRef
     size_t bytes = 0;
     std::vector<void *> blocks;  // what the volumes were allocated as
@@ -246,14 +246,19 @@ int max_zchunk(const Geo3 &g)
     return (int)std::min<long long>(1 << 20, (planes - 8) / 4 * 4);
 }
 
-// z-chunk of a launch: `requested` (64 by default) on a large grid; on a
-// small grid a shorter chunk, so that a launch still has about 2048
-// workgroups (8 per CU) to spread over the 256 CUs -- each chunk re-reads a
-// 4-plane halo of sigma_z on either side, which the parallelism pays for
-// below 64 planes -- but never below 8 planes.  `fixed` keeps `requested`.
-// The result is always a multiple of 4 within [4, max_zchunk(g)], so a
-// chunk's planes and halo stay within 32-bit byte offsets; 0 when even 4
-// planes do not.
+// z-chunk of a launch: `requested` on a large grid; on a small grid a shorter
+// chunk, so that a launch still has about 2048 workgroups (8 per CU) to
+// spread over the 256 CUs -- each chunk re-reads a 4-plane halo of sigma_z on
+// either side, which the parallelism pays for below 64 planes -- but never
+// below 8 planes.  `fixed` keeps `requested`.
+// The one-level launches ask for 8 planes: their workgroups run through a
+// chunk in no particular order, and the shorter it is the closer together in
+// memory they all read (step_tile), which pays for the halo: 460 x 572 x 572,
+// forward 942 us at 8 planes, 961 at 4, 955 at 12, 1038 at 64; gradient 2405,
+// 2394, 2446, 2552; RTM 1988, 2137, 1975, 2004; 239 x 283 x 232, forward 97,
+// 101, 98 and 115.  (The whole steps were 1068, 2566, 2087 and 108 us with 64
+// planes, 12 in the smaller volume, and each XCD in a chunk of its own.)  The
+// two-level launches, which step a chunk's halo planes twice, ask for 64.
 int choose_zchunk(const Geo3 &g, int requested, bool fixed)
 {
     const int cap = max_zchunk(g);
@@ -406,21 +411,23 @@ long long dev_index(const Geo3 &g, long long ref_index)
 }
 
 struct Launch {
-    int ntx, nty, ntz;
+    int ntx, nty, zc;
     dim3 grid, block;
 };
 
-Launch launch_shape(const vti3d_prop *p)
+Launch launch_shape(const Geo3 &g, int rows, int zc)
 {
     Launch L;
-    const Geo3 &g = p->g;
     L.ntx = (g.nx - 4 + 63) / 64;
-    L.nty = (g.ny - 8 + kBY - 1) / kBY;
-    L.ntz = (g.zmax + p->zc - 1) / p->zc;
-    L.block = dim3(64, kBY);
-    L.grid = dim3(L.ntx * L.nty * L.ntz);
+    L.nty = (g.ny - 8 + rows - 1) / rows;
+    L.zc = zc;
+    L.block = dim3(64, rows);
+    L.grid = dim3(L.ntx * L.nty * ((g.zmax + zc - 1) / zc));
     return L;
 }
+Launch launch_shape(const vti3d_prop *p) { return launch_shape(p->g, kBY, p->zc); }
+// 64 x 16 tiles of the two-level kernel
+Launch launch_shape_t2(const vti3d_prop *p) { return launch_shape(p->g, 16, p->zc2); }
 
 // Whether a step that touches this many float volumes streams what it reads or
 // writes once a point past the caches.  Well above the 288 MB that the Infinity
@@ -439,7 +446,7 @@ void fwd_kernel(vti3d_prop *p, const Launch &L, long long src_dev, float src_val
 {
     hipLaunchKernelGGL((vti::fwd3d_kernel<ARITH, ABC, kBY, NT>), L.grid, L.block, 0, p->ctx->stream, p->sx[1],
                        p->sx[0], p->sz[1], p->sz[0], p->cm[p->active][0], p->cm[p->active][1], p->cm[p->active][2],
-                       p->dxy, p->dzv, p->g, p->zc, L.ntx, L.nty, p->dt2dx2, p->dt2dy2, p->dt2dz2, src_dev, src_val);
+                       p->dxy, p->dzv, p->g, L.zc, L.ntx, L.nty, p->dt2dx2, p->dt2dy2, p->dt2dz2, src_dev, src_val);
 }
 
 // f(std::true_type or std::false_type) for a run-time flag
@@ -466,22 +473,12 @@ int fwd_launch(vti3d_prop *p, bool absorbing, long long src_dev, float src_val)
     return vti::kOk;
 }
 
-// 64 x 16 tiles of the two-level kernel
-Launch launch_shape_t2(const vti3d_prop *p)
-{
-    Launch L = launch_shape(p);
-    L.nty = (p->g.ny - 8 + 15) / 16;
-    L.block = dim3(64, 16);
-    L.grid = dim3(L.ntx * L.nty * L.ntz);
-    return L;
-}
-
 template <int ARITH, bool ABC>
 void fwd_t2_kernel(vti3d_prop *p, const Launch &L, long long src_dev, float v1, float v2)
 {
     hipLaunchKernelGGL((vti::fwd3d_t2b_kernel<ARITH, ABC>), L.grid, L.block, 0, p->ctx->stream, p->sx2[0],
                        p->sz2[0], p->sx2[1], p->sz2[1], p->sx[1], p->sz[1], p->sx[0], p->sz[0], p->cm[p->active][0],
-                       p->cm[p->active][1], p->cm[p->active][2], p->dxy, p->dzv, p->g, p->zc, L.ntx, L.nty,
+                       p->cm[p->active][1], p->cm[p->active][2], p->dxy, p->dzv, p->g, L.zc, L.ntx, L.nty,
                        p->dt2dx2, p->dt2dy2, p->dt2dz2, src_dev, v1, v2);
 }
 
@@ -532,7 +529,7 @@ void bwd_kernel(vti3d_prop *p, const Launch &L, long long src_dev, float src_val
                        p->sz[1], p->sz[0], p->lx[1], p->lx[0], p->lz[1], p->lz[0], p->cm[p->active][0],
                        p->cm[p->active][1], p->cm[p->active][2], p->acc[0], MODE == 0 ? p->acc[1] : nullptr,
                        MODE == 0 ? p->acc[2] : nullptr, p->dxy, p->dzv,
-                       p->g, p->zc, L.ntx, L.nty, p->dx2, p->dy2, p->dz2, p->dt2, p->dt2dx2, p->dt2dy2, p->dt2dz2,
+                       p->g, L.zc, L.ntx, L.nty, p->dx2, p->dy2, p->dz2, p->dt2, p->dt2dx2, p->dt2dy2, p->dt2dz2,
                        src_dev, src_val, zrec0, rec);
 }
 
@@ -787,7 +784,11 @@ int vti3d_prop_create(vti_ctx *ctx, vti3d_prop **out, int nx, int ny, int nz, in
     p->dt2dy2 = p->dt2 / p->dy2;
     p->dt2dz2 = p->dt2 / p->dz2;
     const char *zenv = getenv("VTI_ZCHUNK");
-    p->zc = choose_zchunk(g, zenv ? atoi(zenv) : p->zc, zenv != nullptr);
+    p->zc = choose_zchunk(g, zenv ? atoi(zenv) : 8, zenv != nullptr);
+    // below 4 workgroups a CU, 4 planes (100 x 100 x 100: forward 12.2 us a level against 14.9, gradient 23 against
+    // 27; 163 x 140 x 128: 24.1 against 25.7, 49 against 52, RTM 46.6 against 47.6; 200 x 220 x 210, 11 a CU: slower)
+    if (!zenv && p->zc == 8 && launch_shape(g, kBY, 8).grid.x < 1024) p->zc = 4;
+    p->zc2 = choose_zchunk(g, zenv ? atoi(zenv) : 64, zenv != nullptr);
     if (p->zc == 0) {
         delete p;
         VTI_CHECK(false, "vti3d_prop_create: x-y plane %dx%d too large for 32-bit chunk offsets", nx, ny);
@@ -842,7 +843,7 @@ int vti3d_prop_set_zchunk(vti3d_prop *p, int zc)
     VTI_CHECK(p && zc >= 4 && zc % 4 == 0, "vti3d_prop_set_zchunk: chunk must be a positive multiple of 4");
     VTI_CHECK(zc <= max_zchunk(p->g), "vti3d_prop_set_zchunk: chunk %d above %d for this plane size", zc,
               max_zchunk(p->g));
-    p->zc = zc;
+    p->zc = p->zc2 = zc;
     return vti::kOk;
 }
 

@@ -34,15 +34,27 @@ struct Geo3 {
     long long plane;  // pitch*ny
 };
 
-// Maps the hardware block order (round-robin over the 8 XCDs) to a logical
-// tile order in which each XCD owns a contiguous range of tiles, so halo
-// re-reads between neighbouring tiles hit the same L2.
-__device__ __forceinline__ int xcd_logical_block(int nblocks)
+// The tile and z-chunk of a workgroup.  Blocks go to the 8 XCDs in turn; XCD k
+// takes the k-th eighth of the tiles of every chunk, in order, so that halo
+// re-reads between neighbouring tiles hit the same L2 and all XCDs are at work
+// on the same planes.  What bounds the steps of large volumes is how memory is
+// read: a kernel with the forward step's nine streams and no arithmetic takes
+// 1.06 ms at 460 x 572 x 572 in the order of tiles marching through 64 planes
+// with each XCD in a chunk of its own, 0.97 in chunks of 8 in this order, and
+// 0.86 plane by plane.
+// (A chunk's number of tiles need not be a multiple of 8: the XCDs that get one
+// more than the others are those that the chunk's blocks begin with, other ones
+// in each chunk.)
+__device__ __forceinline__ void step_tile(int ntx, int nty, int &bx, int &by, int &bz)
 {
-    const int i = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-    const int q = nblocks >> 3, r = nblocks & 7;
-    const int xcd = i & 7, pos = i >> 3;
-    return (xcd < r) ? xcd * (q + 1) + pos : r * (q + 1) + (xcd - r) * q + pos;
+    const int n = ntx * nty, i = blockIdx.x, x = i & 7;
+    bz = i / n;
+    const int first = (bz * n) & 7, more = n & 7;  // XCDs first .. first + more - 1 (mod 8) have one more
+    const int before = first + more <= 8 ? min(max(x - first, 0), more)
+                                         : min(x, first + more - 8) + max(x - first, 0);
+    const int tile = x * (n >> 3) + before + ((i - bz * n) >> 3);
+    bx = tile % ntx;
+    by = tile / ntx;
 }
 
 // Raw buffer access (buffer_load/store_dword): a wave-uniform 128-bit
@@ -335,8 +347,8 @@ __global__ __launch_bounds__(64 * BY) void fwd3d_kernel(
     constexpr int R = Tile<BY>::R;
     __shared__ float tile[2][R * W];
 
-    const int lb = xcd_logical_block(gridDim.x * gridDim.y * gridDim.z);
-    const int bx = lb % ntx, by = (lb / ntx) % nty, bz = lb / (ntx * nty);
+    int bx, by, bz;
+    step_tile(ntx, nty, bx, by, bz);
     const int tx = threadIdx.x, ty = threadIdx.y;
     const int x0 = bx * 64, y0 = 4 + by * BY;
     const int zs = bz * zc;
@@ -557,8 +569,8 @@ __global__ __launch_bounds__(1024) void fwd3d_t2b_kernel(
     __shared__ float rq[9][NRIM];   // sigma_z(L) queues of the rim columns, slot = plane mod 9
     __shared__ float q1s[9][S::NT];  // sigma_z(L+1) queues of the tile columns, slot = plane mod 9
 
-    const int lb = xcd_logical_block(gridDim.x * gridDim.y * gridDim.z);
-    const int bxi = lb % ntx, byi = (lb / ntx) % nty, bzi = lb / (ntx * nty);
+    int bxi, byi, bzi;
+    step_tile(ntx, nty, bxi, byi, bzi);
     const int tid = threadIdx.x + 64 * threadIdx.y;
     const int x0 = bxi * 64, y0 = 4 + byi * BY;
     const int zs = bzi * zc, ze = min(zs + zc, g.zmax);
@@ -842,8 +854,8 @@ __global__ __launch_bounds__(64 * BY) __attribute__((amdgpu_waves_per_eu(4))) vo
     __shared__ Inject rec;  // waits here for the end: the march is short of scalar registers
     if (threadIdx.x == 0 && threadIdx.y == 0) rec = rec_arg;
 
-    const int lb = xcd_logical_block(gridDim.x * gridDim.y * gridDim.z);
-    const int bx = lb % ntx, by = (lb / ntx) % nty, bz = lb / (ntx * nty);
+    int bx, by, bz;
+    step_tile(ntx, nty, bx, by, bz);
     const int tx = threadIdx.x, ty = threadIdx.y;
     const int x0 = bx * 64, y0 = 4 + by * BY;
     const int zs = bz * zc;
