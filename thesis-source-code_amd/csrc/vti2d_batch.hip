@@ -1602,11 +1602,22 @@ int vti2d_batch_tune(vti_ctx *ctx, const int *shots, int ns, const int *rloc, in
     double obj = 0;
     const int wave = cache_wave(shots, ns, npad, nz);
     int bl = 2, br = 16, bw = wave >= ns ? 0 : wave;
+    // Shots that fit the chip run resident in the shape (2, 16), which wins at
+    // full length: 22 batches of 2 to 9 shots, 95 to 700 columns wide and 82 to
+    // 511 deep, took 1.2 to 1.8 times as long on the per-level kernels.  A trial
+    // this short shows mostly what a call sets up, and has picked another shape
+    // (5 shots of 232-286 columns, 361 levels: 6.0 ms a call, resident 3.2).
+    bool resident = hipSetDevice(ctx->device) == hipSuccess;
+    for (int s = 0; s < ns && resident; ++s) {
+        const int nnx = shots[6 * s + 1] + 2 * npad;
+        resident = vti::res_fits(&nnx, 1, nnz, true, 0);
+    }
     double best = 1e300;
     for (int lv = 1; lv <= 2; ++lv)
         for (int rows : {8, 16})
             for (int wv : {bw}) {
                 if (lv == 1 && rows != 8) continue;  // the tile height only shapes two-level launches
+                if (resident && (lv == 1 || rows != 16)) continue;
                 VTI_HIP(hipStreamSynchronize(ctx->stream));
                 const auto t0 = std::chrono::steady_clock::now();
                 const int rc = vti2d_objfunc_gradient_batch(ctx, &obj, gc.data(), gc.data() + g, gc.data() + 2 * g,
