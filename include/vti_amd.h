@@ -358,6 +358,8 @@ int vti2d_batch_plan_destroy(vti2d_batch_plan *plan);
  * (24 snapshot intervals) of the same shots on a synthetic model over levels
  * per launch (1, 2) and tile rows (8, 16), and returns the fastest in
  * *levels, *tile_rows (and its trial time in *best_ms when not NULL).
+ * Where every shot fits the chip (vti2d_objfunc_gradient_batch) only the shape
+ * that runs them resident, (2, 16), is timed and returned.
  * *max_wave is modelled, not timed: the most shots whose adjoint working set
  * (16 FP32 planes per shot) fits 192 MB of the Infinity Cache, or 0 when all
  * shots do.  Cached per geometry for the life of the process.  No
