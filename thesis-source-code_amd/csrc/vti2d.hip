@@ -705,7 +705,7 @@ int rtm2d(vti_ctx *ctx, int nhx, float *image, const float *data, const float *c
 
         // ---- source side (rtm_f.cu:110-150)
         const vti::Res2dShot rs = res_shot(c, s, rloc, F, tr.p);
-        bool by_level = !(std_taper && vti::res2d_fits_slices(rs));
+        bool by_level = !(ctx->resident && std_taper && vti::res2d_fits_slices(rs));
         if (!by_level) rc = vti::res2d_slices(rs, wavelet, !odcig, slices.p, &by_level);
         if (!rc) rc = zero2(c, F.p, F.q);
         if (rc) return rc;
@@ -730,7 +730,7 @@ int rtm2d(vti_ctx *ctx, int nhx, float *image, const float *data, const float *c
         VTI_HIP(hipGetLastError());
 
         // ---- receiver side and imaging (rtm_f.cu:152-216)
-        by_level = odcig || !(std_taper && vti::res2d_fits_image(rs));
+        by_level = odcig || !(ctx->resident && std_taper && vti::res2d_fits_image(rs));
         if (!by_level) {
             rc = vti::res2d_image(rs, c.ntNeg, c.nnt_data - 1, slices.p, img.p, &by_level);
             if (!rc && by_level) VTI_HIP(hipMemsetAsync(img.p, 0, n * nh * 4, st));
@@ -868,7 +868,7 @@ int fg2d(vti_ctx *ctx, bool born, float *objfunc, float *gc11, float *gc13, floa
         if (rc) return rc;
 
         const vti::Res2dShot rs = res_shot(c, s, rloc, F, bg.p);
-        bool by_level = !(std_taper && vti::res2d_fits_gn(rs));
+        bool by_level = !(ctx->resident && std_taper && vti::res2d_fits_gn(rs));
         if (!by_level) {
             const float *dcp[3] = {dc[0].p, dc[1].p, dc[2].p};
             rc = vti::res2d_gn(rs, dcp, wavelet, snap.p, acc[0].p, acc[1].p, acc[2].p, &by_level);

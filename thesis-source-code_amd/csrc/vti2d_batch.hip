@@ -163,6 +163,7 @@ struct ShotIn {
 
 // The call's checked arguments and derived sizes.
 struct BatchArgs {
+    bool resident = true;  // the context lets passes run resident
     int ns, nr, NX, nz, nt, npad, NNX, nnz, ratio, nnt, nnt_data, levels, BYT, snap_fmt;
     bool half;
     bool res = false;  // the waves run resident (vti2d_res.h)
@@ -945,7 +946,10 @@ std::vector<std::pair<int, int>> split_waves(const BatchArgs &a, int max_wave, l
 
 // Whether the call's shape arguments leave the launch form to the library:
 // the default, two levels per launch with 16-row tiles.
-bool res_wanted(const BatchArgs &a) { return a.levels == 2 && a.BYT == 16 && (a.snap_fmt == 0 || a.snap_fmt == 3); }
+bool res_wanted(const BatchArgs &a)
+{
+    return a.resident && a.levels == 2 && a.BYT == 16 && (a.snap_fmt == 0 || a.snap_fmt == 3);
+}
 
 // The waves of a call: resident ones (a.res is set) when every shot fits the
 // chip, as many consecutive shots as fit it together and at most max_res
@@ -1109,6 +1113,7 @@ int vti2d_objfunc_gradient_batch(vti_ctx *ctx, double *objfunc, double *gc11, do
               "vti2d_objfunc_gradient_batch: null argument");
     BatchArgs a;
     int rc = parse_args(a, shots, ns, rloc, nr, NX, nz, nt, npad, dx, dz, dt, rate, levels, tile_rows, snap_fmt);
+    a.resident = ctx->resident;
     if (rc) return rc;
     VTI_HIP(hipSetDevice(ctx->device));
     (void)hipGetLastError();
@@ -1148,6 +1153,7 @@ int vti2d_batch_plan_create(vti_ctx *ctx, vti2d_batch_plan **plan, const float *
     auto *pl = new vti2d_batch_plan;
     pl->ctx = ctx;
     int rc = parse_args(pl->a, shots, ns, rloc, nr, NX, nz, nt, npad, dx, dz, dt, rate, levels, tile_rows, snap_fmt);
+    pl->a.resident = ctx->resident;
     hipStream_t st = ctx->stream;
     if (!rc) {
         const hipError_t e = hipSetDevice(ctx->device);
@@ -1377,6 +1383,7 @@ int synth2d_batched(vti_ctx *ctx, float *out, const float *c11, const float *c13
     BatchArgs a;
     int rc = parse_args(a, shots.data(), ns, rl.data(), (int)(rl.size() / 2), nx, nz, nt, npad, dx, dz, dt, rate, 2,
                         16, 0);
+    a.resident = ctx->resident;
     if (rc) return rc;
     VTI_HIP(hipSetDevice(ctx->device));
     hipStream_t st = ctx->stream;
@@ -1495,6 +1502,7 @@ int grad2d_merged(vti_ctx *ctx, const Grad2dPart *p, int n, const float *wavelet
         BatchArgs a;
         int rc = parse_args(a, shots.data(), ns, rl.data(), (int)(rl.size() / 2), NNX - 2 * npad, nz, nt, npad, dx,
                             dz, dt, rate, 2, 16, snap_fmt);
+        a.resident = ctx->resident;
         if (rc) return rc;
         VTI_HIP(hipSetDevice(ctx->device));
         hipStream_t st = ctx->stream;
@@ -1607,7 +1615,7 @@ int vti2d_batch_tune(vti_ctx *ctx, const int *shots, int ns, const int *rloc, in
     // 511 deep, took 1.2 to 1.8 times as long on the per-level kernels.  A trial
     // this short shows mostly what a call sets up, and has picked another shape
     // (5 shots of 232-286 columns, 361 levels: 6.0 ms a call, resident 3.2).
-    bool resident = hipSetDevice(ctx->device) == hipSuccess;
+    bool resident = ctx->resident && hipSetDevice(ctx->device) == hipSuccess;
     for (int s = 0; s < ns && resident; ++s) {
         const int nnx = shots[6 * s + 1] + 2 * npad;
         resident = vti::res_fits(&nnx, 1, nnz, true, 0);

@@ -55,6 +55,7 @@ bool res_fits(const int *nnx, int ns, int nnz, bool grad, int snap_fmt)
 
 bool res2d_fits(vti_ctx *ctx, int nnx, int nnz, bool grad)
 {
+    if (!ctx->resident) return false;
     if (hipSetDevice(ctx->device) != hipSuccess) {
         (void)hipGetLastError();
         return false;

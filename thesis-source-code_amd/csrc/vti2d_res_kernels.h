@@ -51,7 +51,7 @@ namespace vti {
 typedef unsigned long long u64;
 
 // the longest wait for a neighbour's word, in ticks of the 100 MHz wall clock
-constexpr long long kResWait = 50000000LL;
+constexpr long long kResWait = 5000000LL;
 constexpr int kResNW = 4;  // wavefronts of a workgroup, one per SIMD
 
 // LDS planes and strips of tiles of 4 NR rows.  Words of a tile's strips at
