@@ -3,6 +3,8 @@ chip) against the per-level kernels, which `levels=1` asks for: the same bits
 at the edges of their tiles (64 columns, 4 rows to a wavefront's 6), for ragged
 last tiles, with several receivers in one column, in waves of several shots,
 and through the fallback for a grid that does not fit the chip."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -10,6 +12,16 @@ from common2d import args2d, layered2d, problem2d
 from common3d import cij_from, ricker
 
 pytestmark = pytest.mark.gpu
+
+
+def _probe(vti, ctx, rows=0, raised=0):
+    """Has the next passes take `rows` rows a wavefront (0: the fastest) and the
+    `raised`th of them start with its abort flag raised (0: none); returns the
+    passes launched since the last call, the runs that gave up and the row
+    counts that ran."""
+    seen = (ctypes.c_int * 3)()
+    assert vti.lib.vti_ctx_resident_probe(ctx.h, rows, raised, seen) == 0
+    return seen[0], seen[1], {r for r in range(8) if seen[2] >> r & 1}
 
 
 def _shots(widths, nz, npad, nt, vertical=False, seed=1):
@@ -76,3 +88,21 @@ def test_resident_product_and_image_vs_oracle(vti, orc, ctx, nx, nz, npad, nt):
     data = (1e-7 * np.random.default_rng(3).standard_normal(((nt - 1) // 4 + 1, P["nr"]))).astype(np.float32)
     img = vti.rtm2d(ctx, data, *P["c"], P["w"], P["sloc"], P["rloc"], P["taper"], *a)
     assert np.array_equal(img, orc.rtm2d(orc.F32, data, *P["c"], P["w"], P["sloc"], P["rloc"], P["taper"], *a))
+
+
+@pytest.mark.parametrize("max_wave,raised", [(0, 1), (2, 2)])
+def test_plan_runs_resident_again_after_giving_up(vti, ctx, max_wave, raised):
+    """A plan's run that gives up (in its first wave, in its second) falls back
+    to the per-level kernels, and its next run is resident again: same bits."""
+    data, c, w, shots, rloc, rest = _shots((70, 61, 90), 12, 5, 61)
+    print("resident plan giving up", max_wave, raised, flush=True)
+    f0, g0 = vti.objfunc_gradient2d_batch(ctx, data, *c, w, shots, rloc, *rest, levels=1)
+    assert g0.any()
+    waves = 1 if max_wave == 0 else 3
+    with vti.BatchPlan(ctx, data, w, shots, rloc, *rest, max_wave=max_wave) as plan:
+        for k in range(3):
+            _probe(vti, ctx, raised=raised if k == 1 else 0)
+            f1, g1 = plan.run(*c)
+            passes, gone, _ = _probe(vti, ctx)
+            assert f0 == f1 and np.array_equal(g0, g1)
+            assert passes == 2 * waves and gone == (1 if k == 1 else 0)

@@ -163,7 +163,7 @@ struct ShotIn {
 
 // The call's checked arguments and derived sizes.
 struct BatchArgs {
-    bool resident = true;  // the context lets passes run resident
+    vti_ctx *ctx = nullptr;
     int ns, nr, NX, nz, nt, npad, NNX, nnz, ratio, nnt, nnt_data, levels, BYT, snap_fmt;
     bool half;
     bool res = false;  // the waves run resident (vti2d_res.h)
@@ -455,7 +455,7 @@ int setup_res(BatchWave &W, const BatchArgs &a, const int *rloc, hipStream_t st)
     std::vector<int> r0;
     for (int j = 0; j < W.nw; ++j) r0.push_back(a.in[W.s0 + j].r0);
     res_levels(W.res, a, a.wavelet, a.grad);
-    return W.res.setup(W.sb, a.nnz, a.snap_fmt, rloc, r0.data(), st);
+    return W.res.setup(a.ctx, W.sb, a.nnz, a.snap_fmt, rloc, r0.data(), st);
 }
 
 // Allocate (or, with a pool, view) the wave's device buffers and upload its
@@ -948,7 +948,7 @@ std::vector<std::pair<int, int>> split_waves(const BatchArgs &a, int max_wave, l
 // the default, two levels per launch with 16-row tiles.
 bool res_wanted(const BatchArgs &a)
 {
-    return a.resident && a.levels == 2 && a.BYT == 16 && (a.snap_fmt == 0 || a.snap_fmt == 3);
+    return a.ctx->resident && a.levels == 2 && a.BYT == 16 && (a.snap_fmt == 0 || a.snap_fmt == 3);
 }
 
 // The waves of a call: resident ones (a.res is set) when every shot fits the
@@ -967,7 +967,7 @@ std::vector<std::pair<int, int>> plan_waves(BatchArgs &a, int max_res, int max_w
             while (s1 < a.ns && (max_res <= 0 || s1 - s0 < max_res) &&
                    (s1 == s0 || used + a.shot_bytes(s1) <= budget)) {
                 nnx.push_back(a.in[s1].nx + 2 * a.npad);
-                if (!vti::res_fits(nnx.data(), (int)nnx.size(), a.nnz, a.grad, a.snap_fmt)) break;
+                if (!vti::res_fits(a.ctx, nnx.data(), (int)nnx.size(), a.nnz, a.grad, a.snap_fmt)) break;
                 used += a.shot_bytes(s1++);
             }
             if (s1 == s0) break;
@@ -1113,7 +1113,7 @@ int vti2d_objfunc_gradient_batch(vti_ctx *ctx, double *objfunc, double *gc11, do
               "vti2d_objfunc_gradient_batch: null argument");
     BatchArgs a;
     int rc = parse_args(a, shots, ns, rloc, nr, NX, nz, nt, npad, dx, dz, dt, rate, levels, tile_rows, snap_fmt);
-    a.resident = ctx->resident;
+    a.ctx = ctx;
     if (rc) return rc;
     VTI_HIP(hipSetDevice(ctx->device));
     (void)hipGetLastError();
@@ -1153,7 +1153,7 @@ int vti2d_batch_plan_create(vti_ctx *ctx, vti2d_batch_plan **plan, const float *
     auto *pl = new vti2d_batch_plan;
     pl->ctx = ctx;
     int rc = parse_args(pl->a, shots, ns, rloc, nr, NX, nz, nt, npad, dx, dz, dt, rate, levels, tile_rows, snap_fmt);
-    pl->a.resident = ctx->resident;
+    pl->a.ctx = ctx;
     hipStream_t st = ctx->stream;
     if (!rc) {
         const hipError_t e = hipSetDevice(ctx->device);
@@ -1383,7 +1383,7 @@ int synth2d_batched(vti_ctx *ctx, float *out, const float *c11, const float *c13
     BatchArgs a;
     int rc = parse_args(a, shots.data(), ns, rl.data(), (int)(rl.size() / 2), nx, nz, nt, npad, dx, dz, dt, rate, 2,
                         16, 0);
-    a.resident = ctx->resident;
+    a.ctx = ctx;
     if (rc) return rc;
     VTI_HIP(hipSetDevice(ctx->device));
     hipStream_t st = ctx->stream;
@@ -1502,7 +1502,7 @@ int grad2d_merged(vti_ctx *ctx, const Grad2dPart *p, int n, const float *wavelet
         BatchArgs a;
         int rc = parse_args(a, shots.data(), ns, rl.data(), (int)(rl.size() / 2), NNX - 2 * npad, nz, nt, npad, dx,
                             dz, dt, rate, 2, 16, snap_fmt);
-        a.resident = ctx->resident;
+        a.ctx = ctx;
         if (rc) return rc;
         VTI_HIP(hipSetDevice(ctx->device));
         hipStream_t st = ctx->stream;
@@ -1618,7 +1618,7 @@ int vti2d_batch_tune(vti_ctx *ctx, const int *shots, int ns, const int *rloc, in
     bool resident = ctx->resident && hipSetDevice(ctx->device) == hipSuccess;
     for (int s = 0; s < ns && resident; ++s) {
         const int nnx = shots[6 * s + 1] + 2 * npad;
-        resident = vti::res_fits(&nnx, 1, nnz, true, 0);
+        resident = vti::res_fits(ctx, &nnx, 1, nnz, true, 0);
     }
     double best = 1e300;
     for (int lv = 1; lv <= 2; ++lv)

@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "vti2d_res_kernels.h"
+#include "vti_ctx.h"
 #include "vti_dbuf.h"
 
 namespace vti {
@@ -60,9 +61,9 @@ auto with_rows(int nr, F &&f)
 
 // The row count of the least cost(rows, tiles per CU) among those whose tiles
 // of these shots are all on the current device at once, cap(rows) on a CU;
-// 0 when there is none.
+// 0 when there is none.  only: the one count to look at, 0 for all.
 template <class Cap, class Cost>
-int res_best_rows(const int *nnx, int ns, int nnz, Cap &&cap, Cost &&cost)
+int res_best_rows(const int *nnx, int ns, int nnz, int only, Cap &&cap, Cost &&cost)
 {
     int dev = 0, cus = 0, best = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
@@ -72,6 +73,7 @@ int res_best_rows(const int *nnx, int ns, int nnz, Cap &&cap, Cost &&cost)
     }
     double least = 0;
     for (int nr : {1, 2, 3, 4, 6}) {
+        if (only && nr != only) continue;
         const int th = kResNW * nr;
         long long tiles = 0;
         for (int s = 0; s < ns; ++s) tiles += (long long)((nnx[s] - 8 + 63) / 64) * ((nnz - 8 + th - 1) / th);
@@ -92,10 +94,13 @@ struct ResGate {
     hipEvent_t done = nullptr;
 };
 ResGate &res_gate(int dev);
-void res_clear(const DBuf<u64> &halo, hipStream_t st);
-// clears the strips, then launch(), behind the device's last resident launch
+void res_clear(const DBuf<u64> &halo, int *flag, int value, hipStream_t st);
+// Clears the strips of t and the abort flag, then launch(), behind the
+// device's last resident launch.  flag: null for a pass that goes on from
+// another's results and is void with it.  (It is cleared by every run, not once
+// where it is allocated: a plan's runs share it.)
 template <class Launch>
-int res_launch(const DBuf<u64> &halo, hipStream_t st, Launch &&launch)
+int res_launch(vti_ctx *ctx, const ResTiles &t, int *flag, hipStream_t st, Launch &&launch)
 {
     int dev = 0;
     VTI_HIP(hipGetDevice(&dev));
@@ -105,7 +110,10 @@ int res_launch(const DBuf<u64> &halo, hipStream_t st, Launch &&launch)
         VTI_HIP(hipStreamWaitEvent(st, g.done, 0));
     else
         VTI_HIP(hipEventCreateWithFlags(&g.done, hipEventDisableTiming));
-    res_clear(halo, st);
+    auto &probe = ctx->probe;
+    res_clear(t.halo, flag, flag && probe.raise && --probe.raise == 0, st);
+    ++probe.passes;
+    probe.ran |= 1 << t.nr;
     launch();
     VTI_HIP(hipGetLastError());
     VTI_HIP(hipEventRecord(g.done, st));
@@ -115,9 +123,9 @@ int res_launch(const DBuf<u64> &halo, hipStream_t st, Launch &&launch)
 // The rows per wavefront with which shots of these padded widths (nnz rows
 // each) are all on the current device at once in a pass (adjoint or forward;
 // snap_fmt 0 or 3), the fastest of them; 0 when there is none.
-int res_rows(const int *nnx, int ns, int nnz, bool adjoint, int snap_fmt);
+int res_rows(const vti_ctx *ctx, const int *nnx, int ns, int nnz, bool adjoint, int snap_fmt);
 // whether the shots fit in the forward pass and, with grad, in the adjoint
-bool res_fits(const int *nnx, int ns, int nnz, bool grad, int snap_fmt);
+bool res_fits(const vti_ctx *ctx, const int *nnx, int ns, int nnz, bool grad, int snap_fmt);
 
 // Tables of the shots base (all fields but tile0/ntx as the caller keeps
 // them) in tiles of nr rows a wavefront, and the receivers of each: rxz[2 r0[j]
@@ -130,7 +138,7 @@ int res_setup(ResTiles &t, int nr, const std::vector<ShotB> &base, int nnz, cons
 ResArgs res_args(const ResTiles &t, int *abort, const BatchGeo &bg, float dx2, float dz2, float dt2, const float *c11,
                  const float *c13, const float *c33, const float *t0, float *tr);
 // after the stream is idle: whether a wait ran out
-int res_gave_up(const DBuf<int> &abort, bool *yes, hipStream_t st);
+int res_gave_up(vti_ctx *ctx, const DBuf<int> &abort, bool *yes, hipStream_t st);
 
 template <class T>
 int res_upload(DBuf<T> &d, const std::vector<T> &h, hipStream_t st)
@@ -143,6 +151,7 @@ int res_upload(DBuf<T> &d, const std::vector<T> &h, hipStream_t st)
 
 // One set of shots run resident.
 struct ResRun {
+    vti_ctx *ctx = nullptr;
     ResTiles f, b;
     std::vector<LevF> lf;    // set by the caller before setup
     std::vector<LevelB> lb;  // the same; empty without an adjoint pass
@@ -152,7 +161,8 @@ struct ResRun {
 
     bool active() const { return f.nr > 0; }
     // the tables of both passes (res_setup)
-    int setup(const std::vector<ShotB> &base, int nnz, int snap_fmt, const int *rxz, const int *r0, hipStream_t st);
+    int setup(vti_ctx *c, const std::vector<ShotB> &base, int nnz, int snap_fmt, const int *rxz, const int *r0,
+              hipStream_t st);
     int forward(const BatchGeo &bg, float dx2, float dz2, float dt2, const DBuf<float> *c, const float *t0, float *tr,
                 int nt, bool taper_first, const SnapW &sw, int last_snap, hipStream_t st);
     int adjoint(const BatchGeo &bg, float dx2, float dz2, float dt2, const DBuf<float> *c, const float *t0, float *tr,

@@ -17,8 +17,9 @@ int per_cu(bool adjoint, int snap_fmt)
     return snap_fmt == 3 ? res_per_cu(bwd2d_res_kernel<NR, 3>) : res_per_cu(bwd2d_res_kernel<NR, 0>);
 }
 
-__global__ void zero64_kernel(u64 *__restrict__ p, long long n)
+__global__ void clear_kernel(u64 *__restrict__ p, long long n, int *__restrict__ flag, int value)
 {
+    if (flag && blockIdx.x == 0 && threadIdx.x == 0) *flag = value;
     for (long long k = blockIdx.x * (long long)blockDim.x + threadIdx.x; k < n; k += (long long)gridDim.x * blockDim.x)
         p[k] = 0;
 }
@@ -30,27 +31,27 @@ ResGate &res_gate(int dev)
     return g[dev & 63];
 }
 
-void res_clear(const DBuf<u64> &h, hipStream_t st)
+void res_clear(const DBuf<u64> &h, int *flag, int value, hipStream_t st)
 {
     const unsigned nb = (unsigned)std::max<size_t>(1, std::min<size_t>((h.n + 255) / 256, 4096));
-    hipLaunchKernelGGL(zero64_kernel, dim3(nb), dim3(256), 0, st, h.p, (long long)h.n);
+    hipLaunchKernelGGL(clear_kernel, dim3(nb), dim3(256), 0, st, h.p, (long long)h.n, flag, value);
 }
 
-int res_rows(const int *nnx, int ns, int nnz, bool adjoint, int snap_fmt)
+int res_rows(const vti_ctx *ctx, const int *nnx, int ns, int nnz, bool adjoint, int snap_fmt)
 {
     // us a level takes, from runs of 10 to 984 tiles: the exchange, a
     // wavefront's rows one after the other, and the tiles' traffic
     // (forward 1.50 at 1 row and 56 tiles, 2.81 at 4 and 666, 3.08 at 6 and
     // 450; adjoint 1.64 at 1 and 56, 2.59 at 4 and 407, 3.31 at 6 and 450)
     return res_best_rows(
-        nnx, ns, nnz,
+        nnx, ns, nnz, ctx->probe.rows,
         [&](int nr) { return with_rows(nr, [&](auto n) { return per_cu<n.value>(adjoint, snap_fmt); }); },
         [&](int nr, double t) { return adjoint ? 1.3 + 0.28 * nr + 0.2 * t : 1.15 + 0.22 * nr + 0.38 * t; });
 }
 
-bool res_fits(const int *nnx, int ns, int nnz, bool grad, int snap_fmt)
+bool res_fits(const vti_ctx *ctx, const int *nnx, int ns, int nnz, bool grad, int snap_fmt)
 {
-    return res_rows(nnx, ns, nnz, false, snap_fmt) && (!grad || res_rows(nnx, ns, nnz, true, snap_fmt));
+    return res_rows(ctx, nnx, ns, nnz, false, snap_fmt) && (!grad || res_rows(ctx, nnx, ns, nnz, true, snap_fmt));
 }
 
 bool res2d_fits(vti_ctx *ctx, int nnx, int nnz, bool grad)
@@ -60,7 +61,7 @@ bool res2d_fits(vti_ctx *ctx, int nnx, int nnz, bool grad)
         (void)hipGetLastError();
         return false;
     }
-    return res_fits(&nnx, 1, nnz, grad, 0);
+    return res_fits(ctx, &nnx, 1, nnz, grad, 0);
 }
 
 int res_setup(ResTiles &t, int nr, const std::vector<ShotB> &base, int nnz, const int *rxz, const int *r0,
@@ -131,17 +132,19 @@ ResArgs res_args(const ResTiles &t, int *abort, const BatchGeo &bg, float dx2, f
     return a;
 }
 
-int ResRun::setup(const std::vector<ShotB> &base, int nnz, int snap_fmt, const int *rxz, const int *r0, hipStream_t st)
+int ResRun::setup(vti_ctx *c, const std::vector<ShotB> &base, int nnz, int snap_fmt, const int *rxz, const int *r0,
+                  hipStream_t st)
 {
+    ctx = c;
     std::vector<int> nnx;
     for (const ShotB &b : base) nnx.push_back(b.nnx);
     const int ns = (int)base.size();
-    int rc = res_setup(f, res_rows(nnx.data(), ns, nnz, false, snap_fmt), base, nnz, rxz, r0, st);
+    int rc = res_setup(f, res_rows(ctx, nnx.data(), ns, nnz, false, snap_fmt), base, nnz, rxz, r0, st);
     if (!rc && !lb.empty())
-        rc = res_setup(b, res_rows(nnx.data(), ns, nnz, true, snap_fmt), base, nnz, rxz, r0, st);
+        rc = res_setup(b, res_rows(ctx, nnx.data(), ns, nnz, true, snap_fmt), base, nnz, rxz, r0, st);
     if (!rc) rc = res_upload(lfd, lf, st);
     if (!rc) rc = res_upload(lbd, lb, st);
-    if (!rc) rc = abortd.alloc(1, st);
+    if (!rc) rc = abortd.alloc(1, st, false);
     return rc;
 }
 
@@ -152,7 +155,7 @@ int ResRun::forward(const BatchGeo &bg, float dx2, float dz2, float dt2, const D
     const ResArgs a = res_args(f, abortd.p, bg, dx2, dz2, dt2, c[0].p, c[1].p, c[2].p, t0, tr);
     const dim3 grid((unsigned)f.ntiles), block(64, kResNW);
     const int tf = taper_first ? 1 : 0;
-    return res_launch(f.halo, st, [&] {
+    return res_launch(ctx, f, abortd.p, st, [&] {
         with_rows(f.nr, [&](auto n) {
             if (sw.s16) fwd2d_res_kernel<n.value, 3><<<grid, block, 0, st>>>(a, lfd.p, nt, tf, sw, last_snap);
             else fwd2d_res_kernel<n.value, 0><<<grid, block, 0, st>>>(a, lfd.p, nt, tf, sw, last_snap);
@@ -168,7 +171,7 @@ int ResRun::adjoint(const BatchGeo &bg, float dx2, float dz2, float dt2, const D
     const ResArgs a = res_args(b, abortd.p, bg, dx2, dz2, dt2, c[0].p, c[1].p, c[2].p, t0, tr);
     const dim3 grid((unsigned)b.ntiles), block(64, kResNW);
     const int nlev = (int)lb.size();
-    return res_launch(b.halo, st, [&] {
+    return res_launch(ctx, b, nullptr, st, [&] {
         with_rows(b.nr, [&](auto n) {
             if (snap_fmt == 3)
                 bwd2d_res_kernel<n.value, 3><<<grid, block, 0, st>>>(a, lbd.p, nlev, sr, last_row, g11, g13, g33);
@@ -178,19 +181,20 @@ int ResRun::adjoint(const BatchGeo &bg, float dx2, float dz2, float dt2, const D
     });
 }
 
-int res_gave_up(const DBuf<int> &abort, bool *yes, hipStream_t st)
+int res_gave_up(vti_ctx *ctx, const DBuf<int> &abort, bool *yes, hipStream_t st)
 {
     int h = 0;
     VTI_HIP(hipMemcpyAsync(&h, abort.p, sizeof h, hipMemcpyDeviceToHost, st));
     VTI_HIP(hipStreamSynchronize(st));
     *yes = h != 0;
+    ctx->probe.gave_up += *yes;
     return kOk;
 }
 
 int ResRun::aborted(bool *yes, hipStream_t st) const
 {
     *yes = false;
-    return active() ? res_gave_up(abortd, yes, st) : kOk;
+    return active() ? res_gave_up(ctx, abortd, yes, st) : kOk;
 }
 
 }  // namespace vti

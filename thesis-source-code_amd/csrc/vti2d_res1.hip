@@ -11,7 +11,7 @@ namespace {
 template <class Kernels>
 int rows_for(const Res2dShot &s, Kernels &&per_cu, double per_row, double per_tile)
 {
-    return res_best_rows(&s.nnx, 1, s.nnz, per_cu,
+    return res_best_rows(&s.nnx, 1, s.nnz, s.ctx->probe.rows, per_cu,
                          [&](int nr, double t) { return 1.3 + per_row * nr + per_tile * t; });
 }
 
@@ -65,7 +65,7 @@ struct Pass {
         if (!rc) rc = res_upload(t0, h0, st);
         if (!rc) rc = res_upload(lf, f, st);
         if (!rc) rc = res_upload(lb, b, st);
-        if (!rc) rc = abort.alloc(1, st);
+        if (!rc) rc = abort.alloc(1, st, false);
         if (rc) return rc;
         BatchGeo bg;
         bg.nnz = s.nnz;
@@ -111,7 +111,7 @@ int res2d_gn(const Res2dShot &s, const float *const *dc, const float *wavelet, f
     if (rc) return rc;
     const SnapW sw{snap, nullptr, false};
     const dim3 block(64, kResNW);
-    rc = res_launch(f.t.halo, st, [&] {
+    rc = res_launch(s.ctx, f.t, f.abort.p, st, [&] {
         with_rows(f.t.nr, [&](auto n) {
             born2d_res_kernel<n.value><<<dim3((unsigned)f.t.ntiles), block, 0, st>>>(f.a, dc[0], dc[1], dc[2], f.lf.p,
                                                                                     s.nt, sw, nnt - 1);
@@ -124,15 +124,15 @@ int res2d_gn(const Res2dShot &s, const float *const *dc, const float *wavelet, f
     Pass b;
     rc = b.init(s, rows_back(s, false), {}, lb, 1, false);
     if (rc) return rc;
-    rc = res_launch(b.t.halo, st, [&] {
+    rc = res_launch(s.ctx, b.t, b.abort.p, st, [&] {
         with_rows(b.t.nr, [&](auto n) {
             back2d_res_kernel<n.value, 0><<<dim3((unsigned)b.t.ntiles), block, 0, st>>>(
                 b.a, b.lb.p, (int)lb.size(), snap, nnt - 1, g11, g13, g33);
         });
     });
     bool g1 = false, g2 = false;
-    if (!rc) rc = res_gave_up(f.abort, &g1, st);
-    if (!rc) rc = res_gave_up(b.abort, &g2, st);
+    if (!rc) rc = res_gave_up(s.ctx, f.abort, &g1, st);
+    if (!rc) rc = res_gave_up(s.ctx, b.abort, &g2, st);
     *gone = g1 || g2;
     return rc;
 }
@@ -148,13 +148,13 @@ int res2d_slices(const Res2dShot &s, const float *wavelet, bool scaled, float *s
     int rc = f.init(s, rows_slices(s), lf, {}, 1, false);
     if (rc) return rc;
     const SnapW sw{slices, nullptr, false};
-    rc = res_launch(f.t.halo, st, [&] {
+    rc = res_launch(s.ctx, f.t, f.abort.p, st, [&] {
         with_rows(f.t.nr, [&](auto n) {
             fwd2d_res_kernel<n.value, kResSlice><<<dim3((unsigned)f.t.ntiles), dim3(64, kResNW), 0, st>>>(
                 f.a, f.lf.p, s.nt, 1, sw, -1);
         });
     });
-    return rc ? rc : res_gave_up(f.abort, gone, st);
+    return rc ? rc : res_gave_up(s.ctx, f.abort, gone, st);
 }
 
 int res2d_image(const Res2dShot &s, int nt_neg, int last_row, const float *slices, float *image, bool *gone)
@@ -170,13 +170,13 @@ int res2d_image(const Res2dShot &s, int nt_neg, int last_row, const float *slice
     Pass b;
     int rc = b.init(s, rows_back(s, true), {}, lb, 1, true);
     if (rc) return rc;
-    rc = res_launch(b.t.halo, st, [&] {
+    rc = res_launch(s.ctx, b.t, b.abort.p, st, [&] {
         with_rows(b.t.nr, [&](auto n) {
             back2d_res_kernel<n.value, 1><<<dim3((unsigned)b.t.ntiles), dim3(64, kResNW), 0, st>>>(
                 b.a, b.lb.p, (int)lb.size(), slices, last_row, image, nullptr, nullptr);
         });
     });
-    return rc ? rc : res_gave_up(b.abort, gone, st);
+    return rc ? rc : res_gave_up(s.ctx, b.abort, gone, st);
 }
 
 }  // namespace vti

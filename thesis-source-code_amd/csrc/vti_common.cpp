@@ -229,6 +229,18 @@ int vti_ctx_set_snapshots(vti_ctx *c, int snap_fmt)
     return vti::kOk;
 }
 
+int vti_ctx_resident_probe(vti_ctx *c, int rows, int raise, int *seen)
+{
+    VTI_CHECK(c != nullptr && seen != nullptr && rows >= 0 && raise >= 0, "vti_ctx_resident_probe: bad arguments");
+    seen[0] = c->probe.passes;
+    seen[1] = c->probe.gave_up;
+    seen[2] = c->probe.ran;
+    c->probe = {};
+    c->probe.rows = rows;
+    c->probe.raise = raise;
+    return vti::kOk;
+}
+
 int vti_ctx_synchronize(vti_ctx *c)
 {
     VTI_CHECK(c != nullptr, "null context");

@@ -17,4 +17,20 @@ struct vti_ctx {
     // several, where other slots' launches can keep the workgroups of a
     // resident one from being placed together until its wait runs out
     bool resident = true;
+    // the resident passes' side of vti_ctx_resident_probe
+    struct {
+        int rows = 0;    // rows of a wavefront to take where the shots then fit, 0: the fastest
+        int raise = 0;   // which pass from now on (1: the next) starts with its abort flag raised, 0: none;
+                         // those with a flag of their own count, not an adjoint's, which is its forward pass's
+        int passes = 0;  // launched
+        int gave_up = 0; // runs found void
+        int ran = 0;     // bit r: some pass took r rows
+    } probe;
 };
+
+// For the tests of the resident 2D passes: sets what the next ones do
+// (vti_ctx::probe) and returns in seen[0..2] the passes launched, the runs
+// that gave up and the row counts taken since the last call.  A raised flag
+// is what a pass finds whose wait has run out: every kernel ends as usual, and the
+// host takes the results for void.
+extern "C" int vti_ctx_resident_probe(vti_ctx *ctx, int rows, int raise, int *seen);
