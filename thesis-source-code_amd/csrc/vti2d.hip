@@ -339,11 +339,12 @@ int vti2d_synthetic(vti_ctx *ctx, float *data, const float *c11, const float *c1
     // Several shots with the standard taper (and rate/dt rounding the same in
     // float as in synthetic_f's double) run as one batch, bit for bit; so does one
     // that fits the chip (136 x 120 points: 1.5 us a level resident, 4 us
-    // launch by launch).
+    // launch by launch).  (Looked at before the taper, whose comparison takes 1 ms
+    // for 5 M points.)
     if (ctx && ns >= 1 && data && c11 && c13 && c33 && wavelet && dx > 0 && dz > 0 && dt > 0 &&
         (int)(rate / dt + 0.5f) == (int)(rate / dt + 0.5) &&
-        vti::grad2d_batchable(sloc, ns, rloc, nr, taper, nx, nz, nt, npad, dt, rate, ot) &&
-        (ns >= 2 || vti::res2d_fits(ctx, nx + 2 * npad, nz + 2 * npad, false)))
+        (ns >= 2 || vti::res2d_fits(ctx, nx + 2 * npad, nz + 2 * npad, false)) &&
+        vti::grad2d_batchable(sloc, ns, rloc, nr, taper, nx, nz, nt, npad, dt, rate, ot))
         return vti::synth2d_batched(ctx, data, c11, c13, c33, wavelet, sloc, ns, rloc, nr, nx, nz, nt, npad, dx, dz,
                                     dt, rate);
     Call2 c;
@@ -664,7 +665,10 @@ int rtm2d(vti_ctx *ctx, int nhx, float *image, const float *data, const float *c
     if (rc) return rc;
     // resident passes (vti2d_res1.hip) where the shot fits the chip: 456 x 732
     // points, 2.4 us a level against 4.8-5.5 launch by launch
-    const bool std_taper = standard_taper(c, taper);
+    const vti::Res2dShot grid{ctx, c.g.nnx, c.g.nnz};
+    bool res_source = ctx->resident && vti::res2d_fits_slices(grid);
+    bool res_image = ctx->resident && !odcig && vti::res2d_fits_image(grid);
+    if ((res_source || res_image) && !standard_taper(c, taper)) res_source = res_image = false;
     const dim3 rows((c.g.nnx - 8 + 255) / 256, c.g.nnz - 8);
     const int xlo = odcig ? std::max(4, nhx) : 4;
     const dim3 xrows((std::max(1, c.g.nnx - 2 * xlo) + 255) / 256, c.g.nnz - 8);
@@ -705,7 +709,7 @@ int rtm2d(vti_ctx *ctx, int nhx, float *image, const float *data, const float *c
 
         // ---- source side (rtm_f.cu:110-150)
         const vti::Res2dShot rs = res_shot(c, s, rloc, F, tr.p);
-        bool by_level = !(ctx->resident && std_taper && vti::res2d_fits_slices(rs));
+        bool by_level = !res_source;
         if (!by_level) rc = vti::res2d_slices(rs, wavelet, !odcig, slices.p, &by_level);
         if (!rc) rc = zero2(c, F.p, F.q);
         if (rc) return rc;
@@ -730,7 +734,7 @@ int rtm2d(vti_ctx *ctx, int nhx, float *image, const float *data, const float *c
         VTI_HIP(hipGetLastError());
 
         // ---- receiver side and imaging (rtm_f.cu:152-216)
-        by_level = odcig || !(ctx->resident && std_taper && vti::res2d_fits_image(rs));
+        by_level = !res_image;
         if (!by_level) {
             rc = vti::res2d_image(rs, c.ntNeg, c.nnt_data - 1, slices.p, img.p, &by_level);
             if (!rc && by_level) VTI_HIP(hipMemsetAsync(img.p, 0, n * nh * 4, st));
@@ -842,7 +846,8 @@ int fg2d(vti_ctx *ctx, bool born, float *objfunc, float *gc11, float *gc13, floa
     // the shot fits the chip: 381 x 497 points, 2.7 us a level against 5.4-6.7
     // launch by launch.  (The gradient's shots have come here because they do
     // not.)
-    const bool std_taper = born && standard_taper(c, taper);
+    const bool res_gn = born && ctx->resident && vti::res2d_fits_gn(vti::Res2dShot{ctx, c.g.nnx, c.g.nnz}) &&
+                        standard_taper(c, taper);
     double obj = 0.0;
     std::vector<int> hmap(n, -1);
     for (int is = 0; is < ns; ++is) {
@@ -868,7 +873,7 @@ int fg2d(vti_ctx *ctx, bool born, float *objfunc, float *gc11, float *gc13, floa
         if (rc) return rc;
 
         const vti::Res2dShot rs = res_shot(c, s, rloc, F, bg.p);
-        bool by_level = !(ctx->resident && std_taper && vti::res2d_fits_gn(rs));
+        bool by_level = !res_gn;
         if (!by_level) {
             const float *dcp[3] = {dc[0].p, dc[1].p, dc[2].p};
             rc = vti::res2d_gn(rs, dcp, wavelet, snap.p, acc[0].p, acc[1].p, acc[2].p, &by_level);
@@ -1194,8 +1199,8 @@ int vti2d_objfunc_gradient(vti_ctx *ctx, float *objfunc, float *gc11, float *gc1
     // adjoint level resident, 20.8 us launch by launch).
     if (ctx && ns >= 1 && objfunc && gc11 && gc13 && gc33 && data && c11 &&
         c13 && c33 && wavelet && dx > 0 && dz > 0 &&
-        vti::grad2d_batchable(sloc, ns, rloc, nr, taper, nx, nz, nt, npad, dt, rate, ot) &&
-        (ns >= 2 || ctx->snap_fmt != 0 || vti::res2d_fits(ctx, nx + 2 * npad, nz + 2 * npad, true))) {
+        (ns >= 2 || ctx->snap_fmt != 0 || vti::res2d_fits(ctx, nx + 2 * npad, nz + 2 * npad, true)) &&
+        vti::grad2d_batchable(sloc, ns, rloc, nr, taper, nx, nz, nt, npad, dt, rate, ot)) {
         vti::Grad2dPart part;
         part.c[0] = c11;
         part.c[1] = c13;
