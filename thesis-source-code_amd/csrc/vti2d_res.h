@@ -10,12 +10,21 @@
 #include "vti2d_res_kernels.h"
 #include "vti_ctx.h"
 #include "vti_dbuf.h"
+#include "vti_res_gate.h"
 
 namespace vti {
 
+// The launch shape of a pass: rows per wavefront (0: the shots do not fit the
+// chip), the workgroups that a CU holds for certain, the device's CUs.
+struct ResShape {
+    int nr = 0, per_cu = 0, cus = 0;
+    explicit operator bool() const { return nr > 0; }
+};
+
 // A pass of a resident run: the tiles of its launch.
 struct ResTiles {
-    int nr = 0, ntiles = 0;  // rows per wavefront (0: the shots do not fit the chip), tiles
+    ResShape shape;
+    int ntiles = 0;
     std::vector<ShotB> sb;
     std::vector<int> tile_shot, rec_at;
     std::vector<ResRec> rec;
@@ -59,17 +68,18 @@ auto with_rows(int nr, F &&f)
     }
 }
 
-// The row count of the least cost(rows, tiles per CU) among those whose tiles
+// The shape of the least cost(rows, tiles per CU) among those whose tiles
 // of these shots are all on the current device at once, cap(rows) on a CU;
-// 0 when there is none.  only: the one count to look at, 0 for all.
+// no rows when there is none.  only: the one row count to look at, 0 for all.
 template <class Cap, class Cost>
-int res_best_rows(const int *nnx, int ns, int nnz, int only, Cap &&cap, Cost &&cost)
+ResShape res_best_rows(const int *nnx, int ns, int nnz, int only, Cap &&cap, Cost &&cost)
 {
-    int dev = 0, cus = 0, best = 0;
+    int dev = 0, cus = 0;
+    ResShape best;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
         (void)hipGetLastError();
-        return 0;
+        return best;
     }
     double least = 0;
     for (int nr : {1, 2, 3, 4, 6}) {
@@ -77,63 +87,64 @@ int res_best_rows(const int *nnx, int ns, int nnz, int only, Cap &&cap, Cost &&c
         const int th = kResNW * nr;
         long long tiles = 0;
         for (int s = 0; s < ns; ++s) tiles += (long long)((nnx[s] - 8 + 63) / 64) * ((nnz - 8 + th - 1) / th);
-        if (tiles > (long long)cus * cap(nr)) continue;
+        const int k = cap(nr);
+        if (tiles > (long long)cus * k) continue;
         const double c = cost(nr, (double)tiles / cus);
         if (best && c >= least) continue;
-        best = nr;
+        best = ResShape{nr, k, cus};
         least = c;
     }
     return best;
 }
 
-// Resident launches of one device follow one another, whatever their
-// streams: two that each hold part of the chip would wait for their missing
-// workgroups for ever.  The mutex covers the enqueueing only.
-struct ResGate {
-    std::mutex mu;
-    hipEvent_t done = nullptr;
+struct ResGateHip {
+    using Stream = hipStream_t;
+    using Event = hipEvent_t;
+    static bool make(Event *e) { return hipEventCreateWithFlags(e, hipEventDisableTiming) == hipSuccess; }
+    static bool record(Event e, Stream s) { return hipEventRecord(e, s) == hipSuccess; }
+    static bool wait(Stream s, Event e) { return hipStreamWaitEvent(s, e, 0) == hipSuccess; }
+    static bool done(Event e) { return hipEventQuery(e) != hipErrorNotReady; }
 };
-ResGate &res_gate(int dev);
+ResGate<ResGateHip> &res_gate(int dev);
 void res_clear(const DBuf<u64> &halo, int *flag, int value, hipStream_t st);
-// Clears the strips of t and the abort flag, then launch(), behind the
-// device's last resident launch.  flag: null for a pass that goes on from
+// Clears the strips of t and the abort flag, then launch(), behind those
+// resident launches of the device that it may not run beside.  flag: null for a pass that goes on from
 // another's results and is void with it.  (It is cleared by every run, not once
 // where it is allocated: a plan's runs share it.)
 template <class Launch>
 int res_launch(vti_ctx *ctx, const ResTiles &t, int *flag, hipStream_t st, Launch &&launch)
 {
     int dev = 0;
+    VTI_HIP(hipGetLastError());
     VTI_HIP(hipGetDevice(&dev));
-    ResGate &g = res_gate(dev);
+    auto &g = res_gate(dev);
     std::lock_guard<std::mutex> lk(g.mu);
-    if (g.done)
-        VTI_HIP(hipStreamWaitEvent(st, g.done, 0));
-    else
-        VTI_HIP(hipEventCreateWithFlags(&g.done, hipEventDisableTiming));
+    VTI_CHECK(g.enter(t.ntiles, t.shape.per_cu, t.shape.cus, st), "resident launch: waiting for others failed");
     auto &probe = ctx->probe;
     res_clear(t.halo, flag, flag && probe.raise && --probe.raise == 0, st);
     ++probe.passes;
-    probe.ran |= 1 << t.nr;
+    probe.ran |= 1 << t.shape.nr;
+    (void)hipGetLastError();  // (an event not ready yet)
     launch();
     VTI_HIP(hipGetLastError());
-    VTI_HIP(hipEventRecord(g.done, st));
+    VTI_CHECK(g.leave(), "resident launch: event record failed");
     return kOk;
 }
 
-// The rows per wavefront with which shots of these padded widths (nnz rows
-// each) are all on the current device at once in a pass (adjoint or forward;
-// snap_fmt 0 or 3), the fastest of them; 0 when there is none.
-int res_rows(const vti_ctx *ctx, const int *nnx, int ns, int nnz, bool adjoint, int snap_fmt);
+// The shape in which shots of these padded widths (nnz rows each) are all on
+// the current device at once in a pass (adjoint or forward; snap_fmt 0 or 3),
+// the fastest; no rows when there is none.
+ResShape res_rows(const vti_ctx *ctx, const int *nnx, int ns, int nnz, bool adjoint, int snap_fmt);
 // whether the shots fit in the forward pass and, with grad, in the adjoint
 bool res_fits(const vti_ctx *ctx, const int *nnx, int ns, int nnz, bool grad, int snap_fmt);
 
 // Tables of the shots base (all fields but tile0/ntx as the caller keeps
-// them) in tiles of nr rows a wavefront, and the receivers of each: rxz[2 r0[j]
+// them) in tiles of that shape, and the receivers of each: rxz[2 r0[j]
 // ..] holds shot j's (ix, iz).  Points outside the interior, where the fields
 // stay 0, are left out.  nf: field pairs exchanged; dipole: the point below
 // each receiver is its negative pole.  The host tables stay in place until the
 // stream has read them.
-int res_setup(ResTiles &t, int nr, const std::vector<ShotB> &base, int nnz, const int *rxz, const int *r0,
+int res_setup(ResTiles &t, const ResShape &shape, const std::vector<ShotB> &base, int nnz, const int *rxz, const int *r0,
               hipStream_t st, int nf = 1, bool dipole = false);
 ResArgs res_args(const ResTiles &t, int *abort, const BatchGeo &bg, float dx2, float dz2, float dt2, const float *c11,
                  const float *c13, const float *c33, const float *t0, float *tr);
@@ -159,7 +170,7 @@ struct ResRun {
     DBuf<LevF> lfd;
     DBuf<LevelB> lbd;
 
-    bool active() const { return f.nr > 0; }
+    bool active() const { return f.shape.nr > 0; }
     // the tables of both passes (res_setup)
     int setup(vti_ctx *c, const std::vector<ShotB> &base, int nnz, int snap_fmt, const int *rxz, const int *r0,
               hipStream_t st);

@@ -25,9 +25,9 @@ __global__ void clear_kernel(u64 *__restrict__ p, long long n, int *__restrict__
 }
 }  // namespace
 
-ResGate &res_gate(int dev)
+ResGate<ResGateHip> &res_gate(int dev)
 {
-    static ResGate *g = new ResGate[64];  // outlives static destructors
+    static auto *g = new ResGate<ResGateHip>[64];  // outlives static destructors
     return g[dev & 63];
 }
 
@@ -37,7 +37,7 @@ void res_clear(const DBuf<u64> &h, int *flag, int value, hipStream_t st)
     hipLaunchKernelGGL(clear_kernel, dim3(nb), dim3(256), 0, st, h.p, (long long)h.n, flag, value);
 }
 
-int res_rows(const vti_ctx *ctx, const int *nnx, int ns, int nnz, bool adjoint, int snap_fmt)
+ResShape res_rows(const vti_ctx *ctx, const int *nnx, int ns, int nnz, bool adjoint, int snap_fmt)
 {
     // us a level takes, from runs of 10 to 984 tiles: the exchange, a
     // wavefront's rows one after the other, and the tiles' traffic
@@ -51,7 +51,8 @@ int res_rows(const vti_ctx *ctx, const int *nnx, int ns, int nnz, bool adjoint, 
 
 bool res_fits(const vti_ctx *ctx, const int *nnx, int ns, int nnz, bool grad, int snap_fmt)
 {
-    return res_rows(ctx, nnx, ns, nnz, false, snap_fmt) && (!grad || res_rows(ctx, nnx, ns, nnz, true, snap_fmt));
+    return bool(res_rows(ctx, nnx, ns, nnz, false, snap_fmt)) &&
+           (!grad || bool(res_rows(ctx, nnx, ns, nnz, true, snap_fmt)));
 }
 
 bool res2d_fits(vti_ctx *ctx, int nnx, int nnz, bool grad)
@@ -64,12 +65,12 @@ bool res2d_fits(vti_ctx *ctx, int nnx, int nnz, bool grad)
     return res_fits(ctx, &nnx, 1, nnz, grad, 0);
 }
 
-int res_setup(ResTiles &t, int nr, const std::vector<ShotB> &base, int nnz, const int *rxz, const int *r0,
+int res_setup(ResTiles &t, const ResShape &shape, const std::vector<ShotB> &base, int nnz, const int *rxz, const int *r0,
               hipStream_t st, int nf, bool dipole)
 {
-    VTI_CHECK(nr > 0, "the shots do not fit the chip");
-    const int th = kResNW * nr, ns = (int)base.size();
-    t.nr = nr;
+    VTI_CHECK(shape, "the shots do not fit the chip");
+    const int nr = shape.nr, th = kResNW * nr, ns = (int)base.size();
+    t.shape = shape;
     t.sb = base;
     t.tile_shot.clear();
     for (int j = 0; j < ns; ++j) {
@@ -156,7 +157,7 @@ int ResRun::forward(const BatchGeo &bg, float dx2, float dz2, float dt2, const D
     const dim3 grid((unsigned)f.ntiles), block(64, kResNW);
     const int tf = taper_first ? 1 : 0;
     return res_launch(ctx, f, abortd.p, st, [&] {
-        with_rows(f.nr, [&](auto n) {
+        with_rows(f.shape.nr, [&](auto n) {
             if (sw.s16) fwd2d_res_kernel<n.value, 3><<<grid, block, 0, st>>>(a, lfd.p, nt, tf, sw, last_snap);
             else fwd2d_res_kernel<n.value, 0><<<grid, block, 0, st>>>(a, lfd.p, nt, tf, sw, last_snap);
         });
@@ -167,12 +168,12 @@ int ResRun::adjoint(const BatchGeo &bg, float dx2, float dz2, float dt2, const D
                     float *tr, const SnapR &sr, int snap_fmt, int last_row, float *g11, float *g13, float *g33,
                     hipStream_t st)
 {
-    VTI_CHECK(active() && b.nr && (snap_fmt == 0 || snap_fmt == 3), "resident adjoint: not set up");
+    VTI_CHECK(active() && b.shape && (snap_fmt == 0 || snap_fmt == 3), "resident adjoint: not set up");
     const ResArgs a = res_args(b, abortd.p, bg, dx2, dz2, dt2, c[0].p, c[1].p, c[2].p, t0, tr);
     const dim3 grid((unsigned)b.ntiles), block(64, kResNW);
     const int nlev = (int)lb.size();
     return res_launch(ctx, b, nullptr, st, [&] {
-        with_rows(b.nr, [&](auto n) {
+        with_rows(b.shape.nr, [&](auto n) {
             if (snap_fmt == 3)
                 bwd2d_res_kernel<n.value, 3><<<grid, block, 0, st>>>(a, lbd.p, nlev, sr, last_row, g11, g13, g33);
             else

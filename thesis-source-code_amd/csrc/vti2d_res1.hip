@@ -9,19 +9,19 @@ namespace vti {
 namespace {
 
 template <class Kernels>
-int rows_for(const Res2dShot &s, Kernels &&per_cu, double per_row, double per_tile)
+ResShape rows_for(const Res2dShot &s, Kernels &&per_cu, double per_row, double per_tile)
 {
     return res_best_rows(&s.nnx, 1, s.nnz, s.ctx->probe.rows, per_cu,
                          [&](int nr, double t) { return 1.3 + per_row * nr + per_tile * t; });
 }
 
-int rows_born(const Res2dShot &s)
+ResShape rows_born(const Res2dShot &s)
 {
     return rows_for(
         s, [](int nr) { return with_rows(nr, [](auto n) { return res_per_cu(born2d_res_kernel<n.value>); }); }, 0.4,
         0.6);
 }
-int rows_back(const Res2dShot &s, bool image)
+ResShape rows_back(const Res2dShot &s, bool image)
 {
     return rows_for(
         s,
@@ -32,7 +32,7 @@ int rows_back(const Res2dShot &s, bool image)
         },
         0.25, 0.3);
 }
-int rows_slices(const Res2dShot &s)
+ResShape rows_slices(const Res2dShot &s)
 {
     return rows_for(
         s,
@@ -49,7 +49,7 @@ struct Pass {
     DBuf<LevelB> lb;
     std::vector<float> h0;
     ResArgs a;
-    int init(const Res2dShot &s, int rows, const std::vector<LevF> &f, const std::vector<LevelB> &b, int nf,
+    int init(const Res2dShot &s, const ResShape &shape, const std::vector<LevF> &f, const std::vector<LevelB> &b, int nf,
              bool dipole)
     {
         hipStream_t st = s.ctx->stream;
@@ -61,7 +61,7 @@ struct Pass {
         h0.resize(s.npad + 1);
         taper_profile2d(h0.data(), s.npad);
         h0[s.npad] = 1.f;
-        int rc = res_setup(t, rows, {sb}, s.nnz, s.rxz, &r0, st, nf, dipole);
+        int rc = res_setup(t, shape, {sb}, s.nnz, s.rxz, &r0, st, nf, dipole);
         if (!rc) rc = res_upload(t0, h0, st);
         if (!rc) rc = res_upload(lf, f, st);
         if (!rc) rc = res_upload(lb, b, st);
@@ -94,8 +94,8 @@ LevelB bracket(double data_t, float image_t)
 }  // namespace
 
 bool res2d_fits_gn(const Res2dShot &s) { return rows_born(s) && rows_back(s, false); }
-bool res2d_fits_slices(const Res2dShot &s) { return rows_slices(s) != 0; }
-bool res2d_fits_image(const Res2dShot &s) { return rows_back(s, true) != 0; }
+bool res2d_fits_slices(const Res2dShot &s) { return bool(rows_slices(s)); }
+bool res2d_fits_image(const Res2dShot &s) { return bool(rows_back(s, true)); }
 
 int res2d_gn(const Res2dShot &s, const float *const *dc, const float *wavelet, float *snap, float *g11, float *g13,
              float *g33, bool *gone)
@@ -112,7 +112,7 @@ int res2d_gn(const Res2dShot &s, const float *const *dc, const float *wavelet, f
     const SnapW sw{snap, nullptr, false};
     const dim3 block(64, kResNW);
     rc = res_launch(s.ctx, f.t, f.abort.p, st, [&] {
-        with_rows(f.t.nr, [&](auto n) {
+        with_rows(f.t.shape.nr, [&](auto n) {
             born2d_res_kernel<n.value><<<dim3((unsigned)f.t.ntiles), block, 0, st>>>(f.a, dc[0], dc[1], dc[2], f.lf.p,
                                                                                     s.nt, sw, nnt - 1);
         });
@@ -125,7 +125,7 @@ int res2d_gn(const Res2dShot &s, const float *const *dc, const float *wavelet, f
     rc = b.init(s, rows_back(s, false), {}, lb, 1, false);
     if (rc) return rc;
     rc = res_launch(s.ctx, b.t, b.abort.p, st, [&] {
-        with_rows(b.t.nr, [&](auto n) {
+        with_rows(b.t.shape.nr, [&](auto n) {
             back2d_res_kernel<n.value, 0><<<dim3((unsigned)b.t.ntiles), block, 0, st>>>(
                 b.a, b.lb.p, (int)lb.size(), snap, nnt - 1, g11, g13, g33);
         });
@@ -149,7 +149,7 @@ int res2d_slices(const Res2dShot &s, const float *wavelet, bool scaled, float *s
     if (rc) return rc;
     const SnapW sw{slices, nullptr, false};
     rc = res_launch(s.ctx, f.t, f.abort.p, st, [&] {
-        with_rows(f.t.nr, [&](auto n) {
+        with_rows(f.t.shape.nr, [&](auto n) {
             fwd2d_res_kernel<n.value, kResSlice><<<dim3((unsigned)f.t.ntiles), dim3(64, kResNW), 0, st>>>(
                 f.a, f.lf.p, s.nt, 1, sw, -1);
         });
@@ -171,7 +171,7 @@ int res2d_image(const Res2dShot &s, int nt_neg, int last_row, const float *slice
     int rc = b.init(s, rows_back(s, true), {}, lb, 1, true);
     if (rc) return rc;
     rc = res_launch(s.ctx, b.t, b.abort.p, st, [&] {
-        with_rows(b.t.nr, [&](auto n) {
+        with_rows(b.t.shape.nr, [&](auto n) {
             back2d_res_kernel<n.value, 1><<<dim3((unsigned)b.t.ntiles), dim3(64, kResNW), 0, st>>>(
                 b.a, b.lb.p, (int)lb.size(), slices, last_row, image, nullptr, nullptr);
         });

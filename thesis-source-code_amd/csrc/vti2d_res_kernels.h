@@ -25,8 +25,8 @@
 // level ahead cannot overwrite a word that is still to be read.
 //
 // All workgroups of a launch must be on the chip at once, since they wait for
-// one another: the host launches no more than fit (res_per_cu) and one
-// resident launch per device at a time.  Every wait is bounded: after
+// one another: the host launches no more than fit (res_per_cu), also of
+// several launches at a time (vti_res_gate.h).  Every wait is bounded: after
 // kResWait without its word (something else holds the CUs) a wavefront raises
 // the abort flag and waits no more, the others see the flag and do the same,
 // and the host, which finds it raised, runs the call on the per-level kernels
