@@ -13,10 +13,7 @@ struct vti_ctx {
     // 1 = FP16, 2 = BF16, 3 = S16 (16-bit integers, power-of-two scale per
     // 64 points), for the calls the batched driver can take
     int snap_fmt = 0;
-    // whether 2D passes may run resident: not on the slots of a server with
-    // several, where other slots' launches can keep the workgroups of a
-    // resident one from being placed together until its wait runs out
-    bool resident = true;
+    bool resident = true;  // whether 2D passes may run resident (vti2d_res.h)
     // the resident passes' side of vti_ctx_resident_probe
     struct {
         int rows = 0;    // rows of a wavefront to take where the shots then fit, 0: the fastest

@@ -81,7 +81,6 @@ struct Request {
 }  // namespace
 
 struct vti_server {
-    int slots = 0;
     int device = 0;
     long long budget = 0;
     std::mutex mu;
@@ -190,7 +189,6 @@ void worker(vti_server *s)
 {
     vti_ctx *ctx = nullptr;
     const int crc = vti_ctx_create(&ctx, s->device);
-    if (crc == vti::kOk) ctx->resident = s->slots == 1;
     for (;;) {
         std::unique_lock<std::mutex> lk(s->mu);
         // the oldest request, once it fits beside those in flight (or runs
@@ -346,7 +344,6 @@ int vti_serve_create(vti_server **out, int device, int slots, double budget_byte
     const size_t mfree = vti::device_free_bytes();  // vti_ctx_create made `device` current
     auto *s = new vti_server();
     s->device = device;
-    s->slots = slots;
     s->budget = budget_bytes > 0 ? (long long)budget_bytes : (long long)mfree - (2LL << 30);
     s->upload_ctx = up;
     for (int k = 0; k < slots; ++k) s->workers.emplace_back(worker, s);
