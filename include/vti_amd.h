@@ -52,6 +52,14 @@ int vti_ctx_set_arith(vti_ctx *ctx, int arith);
  * source wavefield from a random boundary), so the setting does not reach
  * them.  No counterpart in the reference. */
 int vti_ctx_set_snapshots(vti_ctx *ctx, int snap_fmt);
+/* Whether 2D passes on ctx may run resident, all levels of a pass in one
+ * launch whose workgroups wait for one another (1, the default), where the
+ * shots fit the chip; 0 keeps them on the per-level kernels, for a device
+ * that other work keeps full: a pass that cannot be placed whole within 50 ms is
+ * given up and its call done by level.  The results are the same bit for bit.
+ * Plans keep the setting they were created with.  No counterpart in the
+ * reference. */
+int vti_ctx_set_resident(vti_ctx *ctx, int on);
 
 /* ---- host helpers (bit-exact restatements of the reference's host code) - */
 
@@ -312,8 +320,9 @@ int vti2d_gn_hessian_vepsdel(vti_ctx *ctx, float *gv, float *geps, float *gdel, 
  * of a two-level workgroup tile, 4, 8 or 16 (0: 16).  Neither changes a bit of
  * the result.  The default shape (two levels, 16 rows) leaves the choice to the
  * library: with FP32 or S16 snapshots, shots that fit the chip (up to about
- * 0.78 M points at once) run resident, all levels of a pass in one launch.  snap_fmt: 0 keeps the imaging snapshots in FP32 (the result
- * then equals the one-shot driver's bit for bit); 1 (FP16) and 2 (BF16)
+ * 0.78 M points at once) run resident, all levels of a pass in one launch;
+ * after vti_ctx_set_resident(ctx, 0) it is that shape for all.
+ * snap_fmt: 0 keeps the imaging snapshots in FP32 (the result then equals the one-shot driver's bit for bit); 1 (FP16) and 2 (BF16)
  * store each snapshot slice scaled by a power of two, 3 (S16) 16-bit
  * integers with a power-of-two scale per 64-point row piece, halving their memory;
  * the gradient then differs at the level the format's rounding sets.  The

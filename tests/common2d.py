@@ -5,8 +5,19 @@ Models live on the padded grid (nnz, nnx), x fastest; sloc holds
 both in padded grid indices, as lib/vti-fwi-2d/gradient-param.cu:30-48
 builds them."""
 import numpy as np
+import pytest
 
 from common3d import cij_from, ricker
+
+
+@pytest.fixture(params=["resident", "by-level"])
+def ctx(vti, request):
+    """For modules whose tests are to hold on either route of a 2D pass: a
+    context that lets it run resident where it fits the chip (as all these small
+    grids do), and one that keeps the per-level kernels."""
+    with vti.Context(0) as c:
+        c.set_resident(request.param == "resident")
+        yield c
 
 
 def layered2d(nnz, nnx, seed=0, vmin=1500.0, vmax=3000.0):

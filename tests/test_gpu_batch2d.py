@@ -6,7 +6,7 @@ the global gradients are equal bit for bit for every launch shape.  With
 import numpy as np
 import pytest
 
-from common2d import layered2d
+from common2d import ctx, layered2d  # noqa: F401 (ctx: both routes)
 from common3d import cij_from, rel, ricker
 
 pytestmark = pytest.mark.gpu
@@ -207,12 +207,12 @@ def test_autotuned_launch_shape(vti, ctx):
 @pytest.mark.parametrize("snap,levels,max_wave",
                          [("fp32", 2, 0), ("fp32", 1, 3), ("bf16", 2, 2), ("s16", 2, 1), ("fp16", 1, 3)])
 def test_graph_plan_replays_equal_direct_calls(vti, ctx, snap, levels, max_wave):
-    """A captured plan (hipGraph of the whole launch sequence) replayed on
-    three models, with other drivers' work and synchronisations between the
+    """A plan (by level: captured, a hipGraph of the whole launch sequence; of
+    resident waves: a few launches) run on three models, with other drivers' work and synchronisations between the
     replays, gives each time the direct batched call's bits on that model --
     also the third replay, back on the first model.  With max_wave > 0 the
-    plan holds several waves, two graphs each, replayed two at a time on two
-    streams through two alternating sets of wavefield, snapshot and trace
+    plan holds several waves (captured: two graphs each), run two at a time on
+    two streams through two alternating sets of wavefield, snapshot and trace
     buffers."""
     B = batch_problem(vti, seed=14, ns=4)
     _say("batch2d plan", snap, "levels", levels, "max_wave", max_wave)

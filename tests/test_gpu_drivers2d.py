@@ -7,7 +7,7 @@ and each result states its error against the FP64 oracle."""
 import numpy as np
 import pytest
 
-from common2d import args2d, problem2d
+from common2d import args2d, ctx, problem2d  # noqa: F401 (ctx: both routes)
 from common3d import rel
 
 pytestmark = pytest.mark.gpu

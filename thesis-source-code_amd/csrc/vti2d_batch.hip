@@ -1577,13 +1577,13 @@ int vti2d_batch_tune(vti_ctx *ctx, const int *shots, int ns, const int *rloc, in
     VTI_CHECK(ratio >= 2 && (nt - 1) % ratio == 0, "vti2d_batch_tune: schedule needs rate/dt >= 2 and "
                                                    "(nt-1) %% (rate/dt) == 0");
     const int nt_t = std::min(nt, 24 * ratio + 1);
-    using Key = std::tuple<int, int, int, int, int, int, long long>;
+    using Key = std::tuple<int, bool, int, int, int, int, int, long long>;
     static std::mutex mu;
     static std::map<Key, std::tuple<int, int, int, double>> cache;
     long long h = 1469598103934665603LL;
     for (int k = 0; k < 6 * ns; ++k) h = (h ^ shots[k]) * 1099511628211LL;
     for (int k = 0; k < 2 * nr; ++k) h = (h ^ rloc[k]) * 1099511628211LL;
-    const Key key{ctx->device, ns, NX, nz, npad, ratio, h};
+    const Key key{ctx->device, ctx->resident, ns, NX, nz, npad, ratio, h};
     {
         std::lock_guard<std::mutex> lk(mu);
         auto it = cache.find(key);

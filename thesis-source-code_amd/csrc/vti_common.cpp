@@ -229,6 +229,13 @@ int vti_ctx_set_snapshots(vti_ctx *c, int snap_fmt)
     return vti::kOk;
 }
 
+int vti_ctx_set_resident(vti_ctx *c, int on)
+{
+    VTI_CHECK(c != nullptr && (on == 0 || on == 1), "vti_ctx_set_resident: on must be 0 or 1");
+    c->resident = on != 0;
+    return vti::kOk;
+}
+
 int vti_ctx_resident_probe(vti_ctx *c, int rows, int raise, int *seen)
 {
     VTI_CHECK(c != nullptr && seen != nullptr && rows >= 0 && raise >= 0, "vti_ctx_resident_probe: bad arguments");

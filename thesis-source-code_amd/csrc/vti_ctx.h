@@ -13,7 +13,7 @@ struct vti_ctx {
     // 1 = FP16, 2 = BF16, 3 = S16 (16-bit integers, power-of-two scale per
     // 64 points), for the calls the batched driver can take
     int snap_fmt = 0;
-    bool resident = true;  // whether 2D passes may run resident (vti2d_res.h)
+    bool resident = true;  // whether 2D passes may run resident (vti2d_res.h), vti_ctx_set_resident
     // the resident passes' side of vti_ctx_resident_probe
     struct {
         int rows = 0;    // rows of a wavefront to take where the shots then fit, 0: the fastest

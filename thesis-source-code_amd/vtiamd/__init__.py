@@ -36,6 +36,7 @@ _SIGS = {
     "vti_ctx_synchronize": (c_int, [P]),
     "vti_ctx_set_arith": (c_int, [P, c_int]),
     "vti_ctx_set_snapshots": (c_int, [P, c_int]),
+    "vti_ctx_set_resident": (c_int, [P, c_int]),
     "vti_init_damping3d": (c_int, [P, c_int, c_int, c_int, c_int]),
     "vti_init_taper2d": (c_int, [P, c_int, c_int, c_int]),
     "vti_vepsdel_to_cij": (c_int, [P, P, P, P, P, P, c_float, c_float, c_float, c_longlong]),
@@ -236,6 +237,11 @@ class Context:
         "fp16", "bf16" or "s16"; 16-bit forms apply to calls the batched
         driver takes (see vti_ctx_set_snapshots)."""
         check(_lib.vti_ctx_set_snapshots(self.h, SNAP_FORMATS[snap]), "vti_ctx_set_snapshots")
+
+    def set_resident(self, on: bool):
+        """Whether 2D passes may run resident, all levels in one launch (default),
+        or keep to the per-level kernels (see vti_ctx_set_resident)."""
+        check(_lib.vti_ctx_set_resident(self.h, int(on)), "vti_ctx_set_resident")
 
     def close(self):
         if self.h:
