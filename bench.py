@@ -308,7 +308,7 @@ def batch_small_2d(vtiamd, ctx, ns=32, seed=5):
 def shot_gradient_2d(vtiamd, ctx, nshots=2, ns_call=32):
     """2D gradients of the cfg2 inversion (512x1024 + 40 boundary, 3000 steps,
     1024 receivers, rate 4 ms; initial model against data of the true model
-    with its 64 anomalies): one shot per call (the one-shot loop), and one call
+    with its 64 anomalies): one shot per call, and one call
     with all 32 shots as the reference's configuration makes it (run as one
     batch inside objfunc_gradient2d): shot-gradients/s of both."""
     from vtiamd import workloads as W

@@ -322,7 +322,8 @@ int vti2d_gn_hessian_vepsdel(vti_ctx *ctx, float *gv, float *geps, float *gdel, 
  * library: with FP32 or S16 snapshots, shots that fit the chip (up to about
  * 0.78 M points at once) run resident, all levels of a pass in one launch;
  * after vti_ctx_set_resident(ctx, 0) it is that shape for all.
- * snap_fmt: 0 keeps the imaging snapshots in FP32 (the result then equals the one-shot driver's bit for bit); 1 (FP16) and 2 (BF16)
+ * snap_fmt: 0 keeps the imaging snapshots in FP32 (the result then equals the
+ * one-shot driver's bit for bit); 1 (FP16) and 2 (BF16)
  * store each snapshot slice scaled by a power of two, 3 (S16) 16-bit
  * integers with a power-of-two scale per 64-point row piece, halving their memory;
  * the gradient then differs at the level the format's rounding sets.  The

@@ -843,9 +843,10 @@ int fg2d(vti_ctx *ctx, bool born, float *objfunc, float *gc11, float *gc13, floa
     auto snap_p = [&](int k) { return snap.p + (size_t)k * 2 * n; };
     auto snap_q = [&](int k) { return snap.p + (size_t)k * 2 * n + n; };
     // the Gauss-Newton product's passes run resident (vti2d_res1.hip) where
-    // the shot fits the chip: 381 x 497 points, 2.7 us a level against 5.4-6.7
-    // launch by launch.  (The gradient's shots have come here because they do
-    // not.)
+    // the shot fits the chip, up to about 0.52 M points (the LDS planes of two
+    // fields: 512 tiles of 4 rows or 256 of 6): 381 x 497 points, 2.7 us a level
+    // against 5.4-6.7 launch by launch.  (A gradient's shots run resident through
+    // the batched driver.)
     const bool res_gn = born && ctx->resident && vti::res2d_fits_gn(vti::Res2dShot{ctx, c.g.nnx, c.g.nnz}) &&
                         standard_taper(c, taper);
     double obj = 0.0;

@@ -35,11 +35,14 @@
 // Per point the arithmetic is that of vti2d_kernels.h, operation for
 // operation, so the results are the per-level kernels' bit for bit.
 //
-// What bounds a level: the exchange (1.1 us between a few tiles; 2.2 us between
-// 450, where the edge words, 512 + 32 NR of them per tile, load the fabric) and a
-// wavefront's own chain of operations (0.2 us a row).  One shot of 592 x 1104
-// points: 2.8 us a forward level, 3.3 us an adjoint level, where the two-level
-// launches take 7.6 us for the pair's mean and the one-level launches 10.4.
+// What bounds a level: at a few tiles the exchange (1.1 of 1.5 us); at several
+// hundred the instructions of the rows.  One shot of 592 x 1104 points takes 2.9 us
+// a forward level (666 tiles of 4 rows) and 3.4 us an adjoint level (450 of 6), where
+// the two-level launches take 7.6 us for the pair's mean and the one-level launches
+// 10.4.  In a probe of these loops at that size the levels took 3.15 and 3.7 us, and
+// 1.9 and 2.55 with the exchange left out.  Scalar registers are short: the
+// row and lane masks and the strips' addresses of three bodies keep 78 of them in
+// vector lanes in the 4-row forward kernel and 119 in the 6-row adjoint.
 #pragma once
 
 #include "vti2d_batch_kernels.h"
